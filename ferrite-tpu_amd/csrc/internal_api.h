@@ -1,0 +1,26 @@
+// Entry points of libferrite_hip.so for the Python package of the same tree alone. They keep the
+// conventions of ferrite_hip.h (device pointers, sizes, a stream; 0 or a FERRITE_ERR_* code;
+// nothing allocated, nothing synchronised), but are no part of its C ABI and change with the
+// package.
+#pragma once
+
+#include <stdint.h>
+
+extern "C" {
+
+/*
+ * The bf16 product for operands the matrix kernel cannot read in place: any M, N, K and
+ * any 2-byte aligned pointers, either operand given transposed (as ferrite_hip_matmul_ex).
+ * Operands whose rows do not start at 16-byte boundaries are first copied into the
+ * workspace with their rows padded to a multiple of 8 elements; the workspace also holds
+ * the K split's partials. It has ferrite_internal_matmul_ragged_workspace(...) bytes (0: none
+ * needed; -1: sizes out of range, an operand of 2^33 elements or more among them), which
+ * depends on the sizes and on the operands' alignment, and is 16-byte aligned; a smaller
+ * one fails with FERRITE_ERR_INVALID_ARGUMENT. Its content need not survive the call.
+ */
+int64_t ferrite_internal_matmul_ragged_workspace(const void* x, const void* y, int64_t m, int64_t n, int64_t k,
+                                                 int x_t, int y_t);
+int ferrite_internal_matmul_ragged(const void* x, const void* y, void* out, int64_t m, int64_t n, int64_t k, int x_t,
+                                   int y_t, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
+}  // extern "C"

@@ -23,6 +23,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "internal_api.h"
 
 namespace ferrite {
 namespace {
@@ -632,14 +633,29 @@ struct OperandTile {
   }
 };
 
+// What the ragged kernel (RAG below) needs beyond the sizes: the operands' row pitches in
+// elements (multiples of 8), the K slices' slab pitch in floats, and whether the output's
+// rows take 16-byte stores.
+struct RagArgs {
+  int ldx, ldy;
+  int64_t slab;
+  int vec_out;
+};
+
 // out[M,N] (or, with a K split, the f32 partial slab of K slice blockIdx.x / tiles)
 // = x . y over this slice. XT: x is given transposed, stored [K,M]; YT: y is given
 // transposed, stored [N,K]. BM = 256 or 128 output rows per workgroup (128 only
 // with a k-contiguous x, whose tile is then the first two 64-row subtiles).
-template <typename TO, bool XT, bool YT, int BM = 256, int SLOTS = 2, int EPI = kEpiNone, int W = 8>
+// RAG: any K, M and N, over operands whose rows start at multiples of 8 elements
+// (packed by pack_rows_kernel where they do not). The last stage is short: a
+// k-contiguous operand's 16-byte chunks past K are sent out of range, the other's
+// descriptor ends at row K, so both read as zeros (a chunk that K cuts holds the
+// packing's zeros); output rows that take no 16-byte stores are written element by
+// element, a wave's 64 columns at a time.
+template <typename TO, bool XT, bool YT, int BM = 256, int SLOTS = 2, int EPI = kEpiNone, int W = 8, bool RAG = false>
 __global__ __launch_bounds__(64 * W, W == 8 ? 2 : 1) void gemm_dma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ y,
                                                           TO* __restrict__ out, int M, int N, int K, int tiles_m,
-                                                          int tiles_n, int kslice, bf16* __restrict__ aux) {
+                                                          int tiles_n, int kslice, bf16* __restrict__ aux, RagArgs rag) {
   typedef Gemm2 G;
   typedef OperandTile<!XT> XTl;
   typedef OperandTile<YT> YTl;
@@ -676,15 +692,16 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 2 : 1) void gemm_dma_kernel(const 
   const int wm0 = W == 8 ? (wave >> 2) * (BM / 2) : (wave >> 1) * 128;
   const int wn0 = W == 8 ? (wave & 3) * 64 : (wave & 1) * 128;
   const int kbeg = slice * kslice;
-  const int nk = min(K - kbeg, kslice) / G::BK;
-  out += (int64_t)slice * M * N;
+  const int nk = (min(K - kbeg, kslice) + (RAG ? G::BK - 1 : 0)) / G::BK;
+  out += RAG ? slice * rag.slab : (int64_t)slice * M * N;
+  const int ldx = RAG ? rag.ldx : XT ? M : K, ldy = RAG ? rag.ldy : YT ? K : N;
 
   // Per-lane DMA offsets; free indices past M or N read as zeros.
   uint32_t xoff[kDmaX], yoff[kDmaY];
 #pragma unroll
-  for (int i = 0; i < kDmaX; ++i) xoff[i] = XTl::dma_off(wave + W * i, lane, XT ? M : K, m0, M);
+  for (int i = 0; i < kDmaX; ++i) xoff[i] = XTl::dma_off(wave + W * i, lane, ldx, m0, M);
 #pragma unroll
-  for (int i = 0; i < kDmaY; ++i) yoff[i] = YTl::dma_off(wave + W * i, lane, YT ? K : N, n0, N);
+  for (int i = 0; i < kDmaY; ++i) yoff[i] = YTl::dma_off(wave + W * i, lane, ldy, n0, N);
   // DMA instruction q (x instructions first, then y) of stage kt. A stage past
   // the slice gets an empty buffer range: its instructions read nothing and
   // write zeros into a slot that no later stage reads.
@@ -692,12 +709,21 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 2 : 1) void gemm_dma_kernel(const 
     char* st = smem + (kt % SLOTS) * kStageBytes;
     const int k0 = kbeg + kt * G::BK;
     const uint32_t range = kt < nk ? 0x7ffffff0u : 0u;
+    const int rem = min(K - k0, G::BK);  // RAG: k left from this stage on, at most a stage
+    // RAG: past K, a row of the k-contiguous form goes on into the next one, and the rows of
+    // the other form end.
+    auto off = [&](bool kcontig, uint32_t o) {
+      return RAG && kcontig && (lane & 7) * 8 >= rem ? 0x80000000u : o;
+    };
+    auto bytes = [&](bool kcontig, int ld, int free0) {
+      return RAG && !kcontig && kt < nk ? (uint32_t)(rem * ld - free0) * 2u : range;
+    };
     if (q < kDmaX) {
-      const u32x4 rx = buffer_rsrc(XT ? x + (int64_t)k0 * M + m0 : x + (int64_t)m0 * K + k0, range);
-      dma16(rx, st + XTl::block_off(wave + W * q), xoff[q]);
+      const u32x4 rx = buffer_rsrc(XT ? x + (int64_t)k0 * ldx + m0 : x + (int64_t)m0 * ldx + k0, bytes(!XT, ldx, m0));
+      dma16(rx, st + XTl::block_off(wave + W * q), off(!XT, xoff[q]));
     } else {
-      const u32x4 ry = buffer_rsrc(YT ? y + (int64_t)n0 * K + k0 : y + (int64_t)k0 * N + n0, range);
-      dma16(ry, st + kXBytes + YTl::block_off(wave + W * (q - kDmaX)), yoff[q - kDmaX]);
+      const u32x4 ry = buffer_rsrc(YT ? y + (int64_t)n0 * ldy + k0 : y + (int64_t)k0 * ldy + n0, bytes(YT, ldy, n0));
+      dma16(ry, st + kXBytes + YTl::block_off(wave + W * (q - kDmaX)), off(YT, yoff[q - kDmaX]));
     }
   };
   constexpr int kDmaWave = kDmaX + kDmaY;  // DMA instructions per wave and stage
@@ -803,6 +829,19 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 2 : 1) void gemm_dma_kernel(const 
         }
       }
     const int mg = m0 + wm0 + 32 * i;
+    if constexpr (RAG) {
+      if (!rag.vec_out) {
+        for (int r = 0; r < min(32, M - mg); ++r)
+#pragma unroll
+          for (int c0 = 0; c0 < YF * 32; c0 += 64) {
+            const int c = c0 + lane, n = n0 + wn0 + c;
+            const TO v = *reinterpret_cast<const TO*>(ep + r * kRowBytes + (((c / kPer) ^ (r & (kCh - 1))) * 16) +
+                                                      (c % kPer) * kEs);
+            if (n < N) out[(int64_t)(mg + r) * N + n] = v;
+          }
+        continue;
+      }
+    }
 #pragma unroll
     for (int rr = 0; rr < 32 / kRowsPerInst; ++rr) {
       const int r = rr * kRowsPerInst + lane / kCh, c = lane % kCh;
@@ -831,8 +870,6 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 2 : 1) void gemm_dma_kernel(const 
   }
 }
 
-// out = sum over the K slices of the f32 partial slabs, in slice order
-// (deterministic), cast to TO. MN % 4 == 0.
 // The part's bf16 MFMA ceiling: every wave streams v_mfma_f32_32x32x16_bf16
 // over eight independent accumulators (a product waits for its own
 // accumulator only every eighth instruction, past the instruction's latency)
@@ -866,15 +903,23 @@ __global__ __launch_bounds__(512, 1) void mfma_ceiling_kernel(float* __restrict_
   if (lane == 0) sink[blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)] = t;
 }
 
+// out = sum over the K slices of the f32 partial slabs, in slice order
+// (deterministic), cast to TO. The slabs are `slab` floats apart (slab % 4 == 0, slab >= mn);
+// the GELU epilogues need mn % 4 == 0.
 template <typename TO, int EPI = kEpiNone>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ part, TO* __restrict__ out,
-                                                                int64_t mn, int slices, bf16* __restrict__ aux) {
+                                                                int64_t mn, int slices, bf16* __restrict__ aux,
+                                                                int64_t slab) {
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= mn) return;
   f32x4 acc = *reinterpret_cast<const f32x4*>(part + i);
   for (int s = 1; s < slices; ++s) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(part + (int64_t)s * mn + i);
+    const f32x4 v = *reinterpret_cast<const f32x4*>(part + (int64_t)s * slab + i);
     acc += v;
+  }
+  if (EPI == kEpiNone && i + 4 > mn) {
+    for (int e = 0; e < (int)(mn - i); ++e) out[i + e] = Elem<TO>::from_f32(acc[e]);
+    return;
   }
   if constexpr (EPI != kEpiNone)
     gelu_epilogue<EPI>(bf16x4{(bf16)acc[0], (bf16)acc[1], (bf16)acc[2], (bf16)acc[3]}, reinterpret_cast<bf16*>(out + i),
@@ -977,7 +1022,7 @@ int launch_gemm_f32_split(const void* x, const void* y, void* out, int64_t M, in
     launch_gemm_f32_slices<float, S>(xf, yf, static_cast<float*>(ws), M, N, K, groups, stream);
     const int64_t mn = M * N;
     hipLaunchKernelGGL((gemm_splitk_reduce_kernel<TO>), dim3((unsigned)cdiv(mn / 4, 256)), dim3(256), 0, stream,
-                       static_cast<const float*>(ws), static_cast<TO*>(out), mn, groups, nullptr);
+                       static_cast<const float*>(ws), static_cast<TO*>(out), mn, groups, nullptr, mn);
   } else {
     launch_gemm_f32_slices<TO, S>(xf, yf, static_cast<TO*>(out), M, N, K, 1, stream);
   }
@@ -1062,7 +1107,7 @@ int launch_gemm_dma_t(const void* x, const void* y, void* out, int64_t M, int64_
       if (int rc = allow_lds((const void*)kern, kLds128, stream, "ferrite_matmul")) return rc;
       hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(G::kThreads), kLds128, stream,
                          static_cast<const bf16*>(x), static_cast<const bf16*>(y), static_cast<TO*>(out), (int)M,
-                         (int)N, (int)K, (int)tiles_m, (int)tiles_n, (int)K, ax);
+                         (int)N, (int)K, (int)tiles_m, (int)tiles_n, (int)K, ax, RagArgs{});
       return check_launch("ferrite_matmul");
     }
   }
@@ -1084,16 +1129,16 @@ int launch_gemm_dma_t(const void* x, const void* y, void* out, int64_t M, int64_
     if (int rc = allow_lds((const void*)kern, kLds, stream, "ferrite_matmul")) return rc;
     hipLaunchKernelGGL(kern, grid, dim3(w4 ? 256 : G::kThreads), kLds, stream, static_cast<const bf16*>(x),
                        static_cast<const bf16*>(y), static_cast<TO*>(out), (int)M, (int)N, (int)K, (int)tiles_m,
-                       (int)tiles_n, kslice, ax);
+                       (int)tiles_n, kslice, ax, RagArgs{});
   } else {
     auto kern = gemm_dma_kernel<float, XT, YT>;
     if (int rc = allow_lds((const void*)kern, kLds, stream, "ferrite_matmul")) return rc;
     hipLaunchKernelGGL(kern, grid, dim3(G::kThreads), kLds, stream, static_cast<const bf16*>(x),
                        static_cast<const bf16*>(y), static_cast<float*>(ws), (int)M, (int)N, (int)K, (int)tiles_m,
-                       (int)tiles_n, kslice, nullptr);
+                       (int)tiles_n, kslice, nullptr, RagArgs{});
     const int64_t mn = M * N;
     hipLaunchKernelGGL((gemm_splitk_reduce_kernel<TO, EPI>), dim3((unsigned)cdiv(mn / 4, 256)), dim3(256), 0, stream,
-                       static_cast<const float*>(ws), static_cast<TO*>(out), mn, slices, ax);
+                       static_cast<const float*>(ws), static_cast<TO*>(out), mn, slices, ax, mn);
   }
   return check_launch("ferrite_matmul");
 }
@@ -1118,8 +1163,189 @@ bool dma_ok(const void* x, const void* y, const void* out, int64_t m, int64_t n,
          fits(yt ? 256 * k * 2 : 64 * n * 2) && cdiv(m, (int64_t)128) * cdiv(n, (int64_t)Gemm2::BN) * 16 <= 0x7fffffff;
 }
 
+// ---------------------------------------------------------------------------
+// Ragged bf16 products: any sizes and 2-byte aligned pointers, on the DMA kernel.
+// ---------------------------------------------------------------------------
+// Against the element-wise loads of gemm_kernel (and a torch transpose before it for a
+// transposed operand), which bound that kernel at 78 TFLOP/s, on one MI355X:
+// 2100 x 1003 x 2050 forward 110.6 -> 5.5 (pack) + 18.4 us; its dx (K = 2050, y transposed)
+// 13.8 + 138.9 -> 8.3 + 24.0 + 7.0 (slabs' sum) us; its dy (x transposed) 14.9 + 138.9 ->
+// 7.3 + 22.6 + 6.2 us. A copy of both operands costs a few us where the product costs tens;
+// reading rows in place at odd offsets would take the DMA, which moves aligned 16 bytes.
+
+// dst[r][c] = src[r][c] for c < cols, zeros from there to the pitch ld (cols rounded up to 8):
+// rows that start at 16-byte boundaries, for operands whose own do not. Memory-bound: one
+// 16-byte store per thread, read as aligned dwords (a row that starts at an odd element reads
+// its first and last element alone), nothing outside the row. The x operand's chunks come
+// first, then the y operand's, so that one launch packs both.
+struct PackJob {
+  const bf16* src;
+  bf16* dst;
+  uint32_t chunks;  // rows * ld / 8; 0: nothing to pack
+  int cols, ld;
+};
+__global__ __launch_bounds__(256) void pack_rows_kernel(PackJob a, PackJob b) {
+  uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  const bool second = i >= a.chunks;
+  if (second) i -= a.chunks;
+  const PackJob& j = second ? b : a;
+  if (i >= j.chunks) return;
+  const uint32_t per_row = (uint32_t)j.ld / 8, row = i / per_row;
+  const int c0 = (int)(i - row * per_row) * 8;
+  const uint16_t* src = reinterpret_cast<const uint16_t*>(j.src) + (int64_t)row * j.cols + c0;
+  u32x4 w = {0u, 0u, 0u, 0u};
+  if (c0 + 8 > j.cols) {
+    for (int e = 0; e < j.cols - c0; ++e) {
+      const uint32_t v = (uint32_t)src[e] << (16 * (e & 1));
+#pragma unroll
+      for (int d = 0; d < 4; ++d) w[d] |= (e >> 1) == d ? v : 0u;
+    }
+  } else if (reinterpret_cast<uintptr_t>(src) & 2) {
+    const uint32_t first = src[0], last = src[7];
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(src + 1);
+    const uint32_t d0 = p[0], d1 = p[1], d2 = p[2];
+    w = u32x4{first | (d0 << 16), (d0 >> 16) | (d1 << 16), (d1 >> 16) | (d2 << 16), (d2 >> 16) | (last << 16)};
+  } else {
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(src);
+    w = u32x4{p[0], p[1], p[2], p[3]};
+  }
+  *reinterpret_cast<u32x4*>(j.dst + (int64_t)i * 8) = w;
+}
+
+// Where a ragged product's operands lie and what its workspace holds: the packed x, the packed
+// y (each 16-byte aligned, absent where the operand's rows are aligned already), the K slices'
+// partial slabs.
+struct RagPlan {
+  bool pack_x, pack_y;
+  int64_t rows_x, cols_x, rows_y, cols_y;
+  RagArgs args;
+  int slices;
+  int64_t off_y, off_part, bytes;
+};
+RagPlan rag_plan(const void* x, const void* y, int64_t M, int64_t N, int64_t K, bool xt, bool yt, int64_t cus) {
+  auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  RagPlan p{};
+  p.rows_x = xt ? K : M;
+  p.cols_x = xt ? M : K;
+  p.rows_y = yt ? N : K;
+  p.cols_y = yt ? K : N;
+  p.args.ldx = (int)(cdiv(p.cols_x, (int64_t)8) * 8);
+  p.args.ldy = (int)(cdiv(p.cols_y, (int64_t)8) * 8);
+  p.pack_x = p.cols_x % 8 != 0 || !a16(x);
+  p.pack_y = p.cols_y % 8 != 0 || !a16(y);
+  p.args.slab = cdiv(M * N, (int64_t)4) * 4;
+  p.slices = pick_bm(M, N, xt, cus) == 128 ? 1 : splitk_slices(M, N, K, cus);
+  p.off_y = p.pack_x ? p.rows_x * p.args.ldx * 2 : 0;
+  p.off_part = p.off_y + (p.pack_y ? p.rows_y * p.args.ldy * 2 : 0);
+  p.bytes = p.off_part + (p.slices > 1 ? p.slices * p.args.slab * (int64_t)sizeof(float) : 0);
+  return p;
+}
+
+// Sizes the ragged kernel's 32-bit offsets reach: as dma_ok, on the padded pitches.
+bool rag_ok(int64_t m, int64_t n, int64_t k, bool xt, bool yt) {
+  auto fits = [](int64_t bytes) { return bytes < 0x7ffffff0; };
+  return m <= 0x7fffff00 && n <= 0x7fffff00 && k <= 0x7fffff00 && fits(xt ? 64 * (m + 8) * 2 : 256 * (k + 8) * 2) &&
+         fits(yt ? 256 * (k + 8) * 2 : 64 * (n + 8) * 2) &&
+         cdiv(m, (int64_t)128) * cdiv(n, (int64_t)Gemm2::BN) * 16 <= 0x7fffffff &&
+         m * (k + 8) / 8 < 0x3fffffff && n * (k + 8) / 8 < 0x3fffffff && k * (m + 8) / 8 < 0x3fffffff &&
+         k * (n + 8) / 8 < 0x3fffffff;
+}
+
+template <typename TO, bool XT, bool YT>
+int launch_gemm_rag_t(const bf16* x, const bf16* y, TO* out, int64_t M, int64_t N, int64_t K, const RagPlan& p,
+                      char* ws, hipStream_t stream) {
+  typedef Gemm2 G;
+  const int64_t cus = cu_count(stream);
+  RagArgs args = p.args;
+  const bool split = p.slices > 1;
+  args.vec_out = N % 8 == 0 && (split || (reinterpret_cast<uintptr_t>(out) & 15) == 0);
+  const int64_t tiles_n = cdiv(N, (int64_t)G::BN);
+  if constexpr (!XT) {
+    if (pick_bm(M, N, XT, cus) == 128) {
+      constexpr int kLds128 = 3 * (2 * GemmXTile::kSubBytes + OperandTile<YT>::kBytes);
+      const int64_t tiles_m = cdiv(M, (int64_t)128);
+      auto kern = gemm_dma_kernel<TO, false, YT, 128, 3, kEpiNone, 8, true>;
+      if (int rc = allow_lds((const void*)kern, kLds128, stream, "ferrite_matmul")) return rc;
+      hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(G::kThreads), kLds128, stream, x, y, out,
+                         (int)M, (int)N, (int)K, (int)tiles_m, (int)tiles_n, (int)cdiv(K, (int64_t)G::BK) * G::BK,
+                         nullptr, args);
+      return check_launch("ferrite_matmul");
+    }
+  }
+  const int64_t tiles_m = cdiv(M, (int64_t)G::BM);
+  const int kslice = (int)(cdiv(cdiv(K, (int64_t)p.slices), (int64_t)G::BK) * G::BK);
+  constexpr int kLds = 2 * (OperandTile<!XT>::kBytes + OperandTile<YT>::kBytes);
+  const dim3 grid((unsigned)(tiles_m * tiles_n * p.slices));
+  auto go = [&](auto kern, auto* dst) {
+    if (int rc = allow_lds((const void*)kern, kLds, stream, "ferrite_matmul")) return rc;
+    hipLaunchKernelGGL(kern, grid, dim3(G::kThreads), kLds, stream, x, y, dst, (int)M, (int)N, (int)K, (int)tiles_m,
+                       (int)tiles_n, kslice, nullptr, args);
+    return check_launch("ferrite_matmul");
+  };
+  if (!split) return go(gemm_dma_kernel<TO, XT, YT, 256, 2, kEpiNone, 8, true>, out);
+  float* part = reinterpret_cast<float*>(ws + p.off_part);
+  if (int rc = go(gemm_dma_kernel<float, XT, YT, 256, 2, kEpiNone, 8, true>, part)) return rc;
+  const int64_t mn = M * N;
+  hipLaunchKernelGGL((gemm_splitk_reduce_kernel<TO>), dim3((unsigned)cdiv(mn, 1024)), dim3(256), 0, stream, part, out,
+                     mn, p.slices, nullptr, args.slab);
+  return check_launch("ferrite_matmul");
+}
+
+template <typename TO>
+int launch_gemm_rag(const void* x, const void* y, void* out, int64_t M, int64_t N, int64_t K, bool xt, bool yt,
+                    RagPlan p, void* ws, hipStream_t stream) {
+  const bf16* xp = static_cast<const bf16*>(x);
+  const bf16* yp = static_cast<const bf16*>(y);
+  char* wp = static_cast<char*>(ws);
+  if (reinterpret_cast<uintptr_t>(out) & 7) p.slices = 1;  // the slabs' sum leaves in 8-byte stores
+  if (p.pack_x || p.pack_y) {
+    bf16* const px = reinterpret_cast<bf16*>(wp);
+    bf16* const py = reinterpret_cast<bf16*>(wp + p.off_y);
+    const PackJob a{xp, px, p.pack_x ? (uint32_t)(p.rows_x * (p.args.ldx / 8)) : 0u, (int)p.cols_x, p.args.ldx};
+    const PackJob b{yp, py, p.pack_y ? (uint32_t)(p.rows_y * (p.args.ldy / 8)) : 0u, (int)p.cols_y, p.args.ldy};
+    hipLaunchKernelGGL(pack_rows_kernel, dim3((unsigned)cdiv((int64_t)a.chunks + b.chunks, (int64_t)256)), dim3(256),
+                       0, stream, a, b);
+    if (int rc = check_launch("ferrite_matmul")) return rc;
+    if (p.pack_x) xp = px;
+    if (p.pack_y) yp = py;
+  }
+  TO* o = static_cast<TO*>(out);
+  if (xt && yt) return launch_gemm_rag_t<TO, true, true>(xp, yp, o, M, N, K, p, wp, stream);
+  if (xt) return launch_gemm_rag_t<TO, true, false>(xp, yp, o, M, N, K, p, wp, stream);
+  if (yt) return launch_gemm_rag_t<TO, false, true>(xp, yp, o, M, N, K, p, wp, stream);
+  return launch_gemm_rag_t<TO, false, false>(xp, yp, o, M, N, K, p, wp, stream);
+}
+
 }  // namespace
 }  // namespace ferrite
+
+extern "C" int64_t ferrite_internal_matmul_ragged_workspace(const void* x, const void* y, int64_t m, int64_t n,
+                                                            int64_t k, int x_t, int y_t) {
+  if (m < 1 || n < 1 || k < 1) return -1;
+  const bool xt = x_t != 0, yt = y_t != 0;
+  if (!ferrite::rag_ok(m, n, k, xt, yt)) return -1;
+  return ferrite::rag_plan(x, y, m, n, k, xt, yt, ferrite::cu_count_of(-1)).bytes;
+}
+
+extern "C" int ferrite_internal_matmul_ragged(const void* x, const void* y, void* out, int64_t m, int64_t n, int64_t k,
+                                              int x_t, int y_t, int out_dtype, void* workspace,
+                                              int64_t workspace_bytes, void* stream) {
+  using namespace ferrite;
+  const char* name = "ferrite_internal_matmul_ragged";
+  if (!valid_dtype(out_dtype))
+    return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": dtype must be FERRITE_F32 or FERRITE_BF16");
+  if (m < 1 || n < 1 || k < 1) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": need M, N, K >= 1");
+  if (!x || !y || !out) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": null pointer");
+  const bool xt = x_t != 0, yt = y_t != 0;
+  if (!rag_ok(m, n, k, xt, yt)) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": operands too large");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const RagPlan p = rag_plan(x, y, m, n, k, xt, yt, cu_count(s));
+  if (p.bytes > 0 && (!workspace || workspace_bytes < p.bytes || (reinterpret_cast<uintptr_t>(workspace) & 15)))
+    return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": needs a 16-byte aligned workspace of " +
+                                                  std::to_string(p.bytes) + " bytes");
+  if (out_dtype == FERRITE_BF16) return launch_gemm_rag<bf16>(x, y, out, m, n, k, xt, yt, p, workspace, s);
+  return launch_gemm_rag<float>(x, y, out, m, n, k, xt, yt, p, workspace, s);
+}
 
 extern "C" int64_t ferrite_hip_matmul_workspace(int64_t m, int64_t n, int64_t k, int in_dtype) {
   if (m < 1 || n < 1 || k < 1) return -1;
@@ -1143,13 +1369,22 @@ extern "C" int ferrite_hip_matmul_ex(const void* x, const void* y, void* out, in
     if (out_dtype == FERRITE_BF16) return launch_gemm_dma<bf16>(x, y, out, m, n, k, xt, yt, workspace, workspace_bytes, s);
     return launch_gemm_dma<float>(x, y, out, m, n, k, xt, yt, workspace, workspace_bytes, s);
   }
+  if (in_dtype == FERRITE_BF16 && !xt && !yt && rag_ok(m, n, k, xt, yt)) {
+    // Aligned rows and a K that is no whole number of 64-deep steps: nothing to pack.
+    RagPlan p = rag_plan(x, y, m, n, k, xt, yt, cu_count(s));
+    if (!p.pack_x && !p.pack_y) {
+      if (!workspace || workspace_bytes < p.bytes || (reinterpret_cast<uintptr_t>(workspace) & 15)) p.slices = 1;
+      if (out_dtype == FERRITE_BF16) return launch_gemm_rag<bf16>(x, y, out, m, n, k, xt, yt, p, workspace, s);
+      return launch_gemm_rag<float>(x, y, out, m, n, k, xt, yt, p, workspace, s);
+    }
+  }
   if (xt || yt)
     return fail(FERRITE_ERR_INVALID_ARGUMENT,
                 "ferrite_hip_matmul: transposed operands need bf16, K % 64 == 0, N % 8 == 0, M % 8 == 0 for a "
                 "transposed x, and 16-byte aligned pointers");
   if (in_dtype == FERRITE_BF16) {
-    // Shapes the DMA kernel does not take (ragged K, unaligned rows or pointers): four waves
-    // of 64 x 64 outputs per 128 x 128 tile (256 x 256 tiles spilled 48 bytes per lane).
+    // Shapes the DMA kernel does not read in place (unaligned rows or pointers), with no
+    // workspace to pack them into: four waves of 64 x 64 outputs per 128 x 128 tile (256 x 256 tiles spilled 48 bytes per lane).
     if (out_dtype == FERRITE_BF16) return launch_gemm<bf16, bf16, 128, 128, 64, 2, 2>(x, y, out, m, n, k, s);
     return launch_gemm<bf16, float, 128, 128, 64, 2, 2>(x, y, out, m, n, k, s);
   }

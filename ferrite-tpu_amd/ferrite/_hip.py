@@ -118,6 +118,15 @@ SIGNATURES: dict[str, tuple] = {
     ),
 }
 
+# Entry points for this package alone; must match csrc/internal_api.h.
+INTERNAL: dict[str, tuple] = {
+    "ferrite_internal_matmul_ragged_workspace": (_c_i64, [_vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int]),
+    "ferrite_internal_matmul_ragged": (
+        _c_int,
+        [_vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _vp, _c_i64, _vp],
+    ),
+}
+
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 
@@ -135,7 +144,7 @@ def lib() -> ctypes.CDLL:
                     "(or __graft_entry__.build()). ferrite has no non-HIP fallback."
                 )
             handle = ctypes.CDLL(LIB_PATH)
-            for name, (res, args) in SIGNATURES.items():
+            for name, (res, args) in (*SIGNATURES.items(), *INTERNAL.items()):
                 fn = getattr(handle, name)
                 fn.restype = res
                 fn.argtypes = args

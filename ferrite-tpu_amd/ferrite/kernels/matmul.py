@@ -29,22 +29,28 @@ def _pick_blocks(m: int, n: int, k: int, bm, bn, bk):
 
 
 def _transposed_ok(work, m: int, n: int, k: int, x_t: bool, tensors) -> bool:
-    """Whether the DMA-fed kernel reads a transposed operand in place (ferrite_hip_matmul_ex's
-    rule): bf16, K % 64 == 0, N % 8 == 0, M % 8 == 0 for a transposed x, 16-byte pointers."""
+    """Whether the DMA-fed kernel takes the operands as they lie (ferrite_hip_matmul_ex's rule
+    for a transposed one): bf16, K % 64 == 0, N % 8 == 0, M % 8 == 0 for a transposed x,
+    16-byte pointers."""
     return (work == torch.bfloat16 and k % 64 == 0 and n % 8 == 0 and (not x_t or m % 8 == 0)
             and all(t.data_ptr() % 16 == 0 for t in tensors))
 
 
 def _mm(xs, ys, m: int, n: int, k: int, x_t: bool, y_t: bool, out_dtype):
     """out[m, n] = op(xs) @ op(ys) on the HIP kernel. xs holds x [m, k], or its transpose [k, m]
-    when x_t; ys holds y [k, n], or [n, k] when y_t. A transposed operand the kernel cannot read
-    in place is transposed into a copy first."""
+    when x_t; ys holds y [k, n], or [n, k] when y_t. bf16 operands of other sizes or alignment
+    than the kernel reads in place go through ferrite_internal_matmul_ragged; a transposed f32
+    operand is transposed into a copy first."""
     work = torch.promote_types(xs.dtype, ys.dtype)
     xs = xs.to(work).contiguous()
     ys = ys.to(work).contiguous()
     kernel_out = out_dtype if out_dtype in (torch.float32, torch.bfloat16) else torch.float32
     out = torch.empty((m, n), dtype=kernel_out, device=xs.device)
-    if (x_t or y_t) and not _transposed_ok(work, m, n, k, x_t, (xs, ys, out)):
+    in_place = _transposed_ok(work, m, n, k, x_t, (xs, ys, out))
+    ragged = work == torch.bfloat16 and not in_place and m and n and k
+    ws_bytes = _hip.lib().ferrite_internal_matmul_ragged_workspace(xs.data_ptr(), ys.data_ptr(), m, n, k, int(x_t),
+                                                              int(y_t)) if ragged else -1
+    if (x_t or y_t) and not in_place and ws_bytes < 0:
         if x_t:
             xs, x_t = xs.t().contiguous(), False
         if y_t:
@@ -52,6 +58,13 @@ def _mm(xs, ys, m: int, n: int, k: int, x_t: bool, y_t: bool, out_dtype):
     if m and n:
         if k == 0:
             out.zero_()
+        elif ws_bytes >= 0:
+            ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=xs.device) if ws_bytes > 0 else None
+            rc = _hip.lib().ferrite_internal_matmul_ragged(
+                xs.data_ptr(), ys.data_ptr(), out.data_ptr(), m, n, k, int(x_t), int(y_t), _hip.dtype_code(kernel_out),
+                _hip.ptr(ws), ws_bytes, _hip.stream_of(xs),
+            )
+            _hip.check(rc, "ferrite_matmul")
         else:
             lib = _hip.lib()
             code = _hip.dtype_code(work)

@@ -347,3 +347,47 @@ def test_mfma_ceiling_runs_its_products(dev, waves, blocks, iters):
     want = iters * 8 * D[rows, 0].sum()
     assert np.all(got == got[0]), "every wave computes the same sum"
     assert abs(got[0] - want) <= 1e-4 * iters * 8 * np.abs(D[rows, 0]).sum() + 1e-6, (got[0], want)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 1),           # one element
+    (3, 264, 72),        # aligned rows, a K of one step and a part of the next: nothing packed
+    (257, 250, 63),      # one short step, odd rows on both sides
+    (130, 513, 65),      # one k past a step
+    (520, 263, 1031),    # K split in two, slabs of an odd size
+    (2000, 2055, 321),   # 128-row tiles (k-contiguous x), ragged row and column edges
+    (264, 1000, 1000),   # K % 8 == 0 but not a whole step
+])
+@pytest.mark.parametrize("x_t,y_t", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_ragged_products(dev, m, n, k, x_t, y_t, shift):
+    """ferrite_internal_matmul_ragged over sizes and base pointers (shift: operands and output start one
+    element past an aligned address) that the in-place kernel does not take: f32 output within the
+    f32 accumulation bound of the f64 product, bf16 output within one ulp more, every element
+    written and none past the output; and the Python wrapper's route to it."""
+    a, b, exact, bound = _exact_case(m, n, k)
+    lib = _hip.lib()
+
+    def shifted(v):
+        flat = torch.empty(v.size + shift, dtype=torch.bfloat16, device=dev)
+        flat[shift:] = to_dev(v, "bf16", dev).reshape(-1)
+        return flat[shift:]
+
+    xs, ys = shifted(a.T.copy() if x_t else a), shifted(b.T.copy() if y_t else b)
+    ws_bytes = lib.ferrite_internal_matmul_ragged_workspace(xs.data_ptr(), ys.data_ptr(), m, n, k, int(x_t), int(y_t))
+    ws = torch.full((ws_bytes // 4 + 1,), float("nan"), device=dev)
+    for dt in (torch.float32, torch.bfloat16):
+        buf = torch.full((m * n + shift + 8,), float("nan"), dtype=dt, device=dev)
+        out = buf[shift : shift + m * n]
+        _hip.check(lib.ferrite_internal_matmul_ragged(xs.data_ptr(), ys.data_ptr(), out.data_ptr(), m, n, k, int(x_t),
+                                                 int(y_t), _hip.dtype_code(dt), ws.data_ptr(), ws_bytes,
+                                                 _hip.stream_of(xs)), "matmul_ragged")
+        torch.cuda.synchronize()
+        got = to_np(out).astype(np.float64).reshape(m, n)
+        assert np.all(np.abs(got - exact) <= bound + (bf16_ulp(exact) if dt == torch.bfloat16 else 0.0))
+        assert torch.isnan(buf[:shift]).all() and torch.isnan(buf[shift + m * n :]).all()
+    from ferrite.kernels.matmul import _mm
+
+    same = _mm(xs.view(k, m) if x_t else xs.view(m, k), ys.view(n, k) if y_t else ys.view(k, n), m, n, k, x_t, y_t,
+               torch.float32)
+    assert np.all(np.abs(to_np(same).astype(np.float64) - exact) <= bound)
