@@ -23,4 +23,15 @@ int64_t ferrite_internal_matmul_ragged_workspace(const void* x, const void* y, i
 int ferrite_internal_matmul_ragged(const void* x, const void* y, void* out, int64_t m, int64_t n, int64_t k, int x_t,
                                    int y_t, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/*
+ * out[M,N] = x[M,K] . bf16(w[K,N]) for bf16 x and out and a float w whose elements are rounded
+ * to bf16 as they are read (model/gpt.py:95-104: the linear layer's cast of its weight), with
+ * M <= 64 rows. With aux, the GELU epilogue: aux <- bf16(x . w), out <- bf16(gelu(aux)).
+ * A workspace of ferrite_internal_linear_f32w_workspace(...) bytes (-1: sizes out of range),
+ * 16-byte aligned, lets a deep K split; with less it does not.
+ */
+int64_t ferrite_internal_linear_f32w_workspace(const void* x, const float* w, int64_t m, int64_t n, int64_t k);
+int ferrite_internal_linear_f32w(const void* x, const float* w, void* out, void* aux, int64_t m, int64_t n, int64_t k,
+                                 void* workspace, int64_t workspace_bytes, void* stream);
+
 }  // extern "C"

@@ -23,7 +23,10 @@
 #include <algorithm>
 
 #include "common.h"
+#include "gelu.h"
 #include "internal_api.h"
+#include "skinny.h"
+#include "splitk.h"
 
 namespace ferrite {
 namespace {
@@ -487,52 +490,8 @@ __global__ __launch_bounds__((BMN == 64 ? 128 : 256) * S, 1) void gemm_f32_slice
 }
 
 // ===========================================================================
-// GELU epilogues (the MLP of model/gpt.py:141: jax.nn.gelu(approximate=True))
+// GELU epilogues (gelu.h)
 // ===========================================================================
-// gelu(u) = u/2 (1 + tanh(z)), z = b (u + c u^3), b = sqrt(2/pi), c = 0.044715,
-// written as u s with s = (1 + tanh z)/2 = 1 / (1 + 2^(-2 z log2 e)): one exp2
-// and one reciprocal instead of a libm tanh (the epilogue runs once per output
-// element, after the products, with nothing to hide it behind), and no
-// cancellation in 1 + tanh z at negative u. gelu'(u) = s + 2 u s (1 - s) b (1 + 3 c u^2).
-// Both in f32 from the bf16-rounded u, as an elementwise pass over the rounded
-// product computes them.
-constexpr int kEpiNone = 0, kEpiGelu = 1, kEpiGeluGrad = 2;
-constexpr float kGeluB = 0.7978845608028654f, kGeluC = 0.044715f;
-constexpr float kGeluE = -2.0f * kGeluB * 1.4426950408889634f;  // -2 b log2(e)
-
-__device__ __forceinline__ float gelu_gate(float u) {  // s = (1 + tanh z) / 2
-  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(kGeluE * (u + kGeluC * u * u * u)));
-}
-__device__ __forceinline__ float gelu_tanh(float u) { return u * gelu_gate(u); }
-__device__ __forceinline__ float gelu_tanh_grad(float u) {
-  const float s = gelu_gate(u);
-  return s + 2.f * u * s * (1.f - s) * kGeluB * (1.f + 3.f * kGeluC * u * u);
-}
-
-// Four consecutive outputs v = bf16(x . y) of one row. kEpiGelu: aux <- v (the
-// pre-activation), out <- bf16(gelu(v)). kEpiGeluGrad: u is the pre-activation
-// (read from aux); out <- bf16(v * gelu'(u)) (v is the incoming gradient).
-__device__ __forceinline__ void gelu_store(const bf16x4& v, bf16* out, bf16* aux) {
-  *reinterpret_cast<bf16x4*>(aux) = v;
-  bf16x4 r;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) r[e] = (bf16)gelu_tanh((float)v[e]);
-  *reinterpret_cast<bf16x4*>(out) = r;
-}
-__device__ __forceinline__ void gelu_grad_store(const bf16x4& v, const bf16x4& u, bf16* out) {
-  bf16x4 r;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) r[e] = (bf16)((float)v[e] * gelu_tanh_grad((float)u[e]));
-  *reinterpret_cast<bf16x4*>(out) = r;
-}
-template <int EPI>
-__device__ __forceinline__ void gelu_epilogue(const bf16x4& v, bf16* out, bf16* aux) {
-  if constexpr (EPI == kEpiGelu)
-    gelu_store(v, out, aux);
-  else
-    gelu_grad_store(v, *reinterpret_cast<const bf16x4*>(aux), out);
-}
-
 // The same epilogue as a pass of its own, for products the DMA kernel does not
 // take: kEpiGelu reads the pre-activation from aux, kEpiGeluGrad the gradient
 // from out (both written there by the plain product).
@@ -903,33 +862,6 @@ __global__ __launch_bounds__(512, 1) void mfma_ceiling_kernel(float* __restrict_
   if (lane == 0) sink[blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)] = t;
 }
 
-// out = sum over the K slices of the f32 partial slabs, in slice order
-// (deterministic), cast to TO. The slabs are `slab` floats apart (slab % 4 == 0, slab >= mn);
-// the GELU epilogues need mn % 4 == 0.
-template <typename TO, int EPI = kEpiNone>
-__global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ part, TO* __restrict__ out,
-                                                                int64_t mn, int slices, bf16* __restrict__ aux,
-                                                                int64_t slab) {
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (i >= mn) return;
-  f32x4 acc = *reinterpret_cast<const f32x4*>(part + i);
-  for (int s = 1; s < slices; ++s) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(part + (int64_t)s * slab + i);
-    acc += v;
-  }
-  if (EPI == kEpiNone && i + 4 > mn) {
-    for (int e = 0; e < (int)(mn - i); ++e) out[i + e] = Elem<TO>::from_f32(acc[e]);
-    return;
-  }
-  if constexpr (EPI != kEpiNone)
-    gelu_epilogue<EPI>(bf16x4{(bf16)acc[0], (bf16)acc[1], (bf16)acc[2], (bf16)acc[3]}, reinterpret_cast<bf16*>(out + i),
-                       aux + i);
-  else if constexpr (sizeof(TO) == 2)
-    *reinterpret_cast<bf16x4*>(out + i) = bf16x4{(bf16)acc[0], (bf16)acc[1], (bf16)acc[2], (bf16)acc[3]};
-  else
-    *reinterpret_cast<f32x4*>(out + i) = acc;
-}
-
 template <typename T, typename TO, int BM, int BN, int BK, int WM, int WN, bool AL>
 void launch_gemm_kernel(const void* x, const void* y, void* out, int64_t M, int64_t N, int64_t K, int64_t tiles,
                         int64_t tiles_n, size_t lds, hipStream_t stream) {
@@ -1163,6 +1095,13 @@ bool dma_ok(const void* x, const void* y, const void* out, int64_t m, int64_t n,
          fits(yt ? 256 * k * 2 : 64 * n * 2) && cdiv(m, (int64_t)128) * cdiv(n, (int64_t)Gemm2::BN) * 16 <= 0x7fffffff;
 }
 
+// Whether a product goes to the skinny kernels: few rows and, where the tiles read the operands
+// in place, where they are faster. A transposed y that the tiles do not read stays refused.
+bool use_skinny(const void* x, const void* y, const void* out, int64_t m, int64_t n, int64_t k, bool xt, bool yt) {
+  if (xt || !skinny_ok(m, n, k)) return false;
+  return dma_ok(x, y, out, m, n, k, xt, yt) ? skinny_better(m, n, k) : !yt;
+}
+
 // ---------------------------------------------------------------------------
 // Ragged bf16 products: any sizes and 2-byte aligned pointers, on the DMA kernel.
 // ---------------------------------------------------------------------------
@@ -1323,6 +1262,9 @@ extern "C" int64_t ferrite_internal_matmul_ragged_workspace(const void* x, const
                                                             int64_t k, int x_t, int y_t) {
   if (m < 1 || n < 1 || k < 1) return -1;
   const bool xt = x_t != 0, yt = y_t != 0;
+  if (!xt && ferrite::skinny_ok(m, n, k))
+    return ferrite::skinny_workspace({x, y, nullptr, nullptr, m, n, k, yt, FERRITE_BF16, FERRITE_BF16,
+                                      ferrite::kEpiNone, nullptr, 0});
   if (!ferrite::rag_ok(m, n, k, xt, yt)) return -1;
   return ferrite::rag_plan(x, y, m, n, k, xt, yt, ferrite::cu_count_of(-1)).bytes;
 }
@@ -1337,14 +1279,35 @@ extern "C" int ferrite_internal_matmul_ragged(const void* x, const void* y, void
   if (m < 1 || n < 1 || k < 1) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": need M, N, K >= 1");
   if (!x || !y || !out) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": null pointer");
   const bool xt = x_t != 0, yt = y_t != 0;
-  if (!rag_ok(m, n, k, xt, yt)) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": operands too large");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (!xt && skinny_ok(m, n, k))
+    return skinny_launch({x, y, out, nullptr, m, n, k, yt, FERRITE_BF16, out_dtype, kEpiNone, workspace, workspace_bytes}, s);
+  if (!rag_ok(m, n, k, xt, yt)) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": operands too large");
   const RagPlan p = rag_plan(x, y, m, n, k, xt, yt, cu_count(s));
   if (p.bytes > 0 && (!workspace || workspace_bytes < p.bytes || (reinterpret_cast<uintptr_t>(workspace) & 15)))
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": needs a 16-byte aligned workspace of " +
                                                   std::to_string(p.bytes) + " bytes");
   if (out_dtype == FERRITE_BF16) return launch_gemm_rag<bf16>(x, y, out, m, n, k, xt, yt, p, workspace, s);
   return launch_gemm_rag<float>(x, y, out, m, n, k, xt, yt, p, workspace, s);
+}
+
+extern "C" int64_t ferrite_internal_linear_f32w_workspace(const void* x, const float* w, int64_t m, int64_t n,
+                                                          int64_t k) {
+  using namespace ferrite;
+  if (k < 1 || n < 1 || !skinny_ok(m, n, k)) return -1;
+  return skinny_workspace({x, w, nullptr, nullptr, m, n, k, false, FERRITE_F32, FERRITE_BF16, kEpiNone, nullptr, 0});
+}
+
+extern "C" int ferrite_internal_linear_f32w(const void* x, const float* w, void* out, void* aux, int64_t m, int64_t n,
+                                            int64_t k, void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace ferrite;
+  const char* name = "ferrite_internal_linear_f32w";
+  if (k < 1 || n < 1 || !skinny_ok(m, n, k))
+    return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": sizes out of range");
+  if (!x || !w || !out) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": null pointer");
+  return skinny_launch({x, w, out, aux, m, n, k, false, FERRITE_F32, FERRITE_BF16, aux ? kEpiGelu : kEpiNone, workspace,
+                        workspace_bytes},
+                       static_cast<hipStream_t>(stream));
 }
 
 extern "C" int64_t ferrite_hip_matmul_workspace(int64_t m, int64_t n, int64_t k, int in_dtype) {
@@ -1365,6 +1328,8 @@ extern "C" int ferrite_hip_matmul_ex(const void* x, const void* y, void* out, in
   if (!x || !y || !out) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_matmul: null pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool xt = x_t != 0, yt = y_t != 0;
+  if (in_dtype == FERRITE_BF16 && use_skinny(x, y, out, m, n, k, xt, yt))
+    return skinny_launch({x, y, out, nullptr, m, n, k, yt, FERRITE_BF16, out_dtype, kEpiNone, workspace, workspace_bytes}, s);
   if (in_dtype == FERRITE_BF16 && dma_ok(x, y, out, m, n, k, xt, yt)) {
     if (out_dtype == FERRITE_BF16) return launch_gemm_dma<bf16>(x, y, out, m, n, k, xt, yt, workspace, workspace_bytes, s);
     return launch_gemm_dma<float>(x, y, out, m, n, k, xt, yt, workspace, workspace_bytes, s);
@@ -1411,6 +1376,9 @@ extern "C" int ferrite_hip_matmul_gelu(const void* x, const void* y, void* out, 
   if (aux == out) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": aux and out must differ");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool xt = x_t != 0, yt = y_t != 0;
+  if (use_skinny(x, y, out, m, n, k, xt, yt))
+    return skinny_launch({x, y, out, aux, m, n, k, yt, FERRITE_BF16, FERRITE_BF16,
+                          mode == FERRITE_GELU ? kEpiGelu : kEpiGeluGrad, workspace, workspace_bytes}, s);
   auto a8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; };
   if (dma_ok(x, y, out, m, n, k, xt, yt) && a8(aux)) {
     if (mode == FERRITE_GELU)

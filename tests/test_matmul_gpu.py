@@ -391,3 +391,47 @@ def test_ragged_products(dev, m, n, k, x_t, y_t, shift):
     same = _mm(xs.view(k, m) if x_t else xs.view(m, k), ys.view(n, k) if y_t else ys.view(k, n), m, n, k, x_t, y_t,
                torch.float32)
     assert np.all(np.abs(to_np(same).astype(np.float64) - exact) <= bound)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 1),
+    (1, 4098, 16),     # two columns per lane, one step, the other waves idle
+    (8, 512, 512),     # a decode step's projection
+    (8, 1537, 512),    # odd rows of w: single columns
+    (31, 40, 77),      # K % 8 != 0: x element by element
+    (32, 4352, 1031),  # two columns per lane, ragged K
+    (33, 65, 2048),    # a second row block of one row, K in four slices of an odd slab
+    (3, 77, 4100),     # eight slices, the last short
+    (8, 4098, 4096),   # slices of two columns per lane
+    (64, 8200, 264),   # two full row blocks, two columns per lane
+    (64, 96, 100),
+])
+@pytest.mark.parametrize("y_t", [False, True])
+def test_few_rows(dev, m, n, k, y_t):
+    """Products of up to 64 rows (csrc/skinny.hip) against the f64 product, y as it is and
+    transposed, with f32 and bf16 output; the float-weight form rounds the weight as a cast does."""
+    a, b, exact, bound = _exact_case(m, n, k)
+    lib, st = _hip.lib(), torch.cuda.current_stream().cuda_stream
+    xs, ys = to_dev(a, "bf16", dev), to_dev(b.T.copy() if y_t else b, "bf16", dev)
+    ws_bytes = lib.ferrite_internal_matmul_ragged_workspace(xs.data_ptr(), ys.data_ptr(), m, n, k, 0, int(y_t))
+    assert (ws_bytes > 0) == (k >= 4096 or (m > 32 and k >= 2048)) or n > 4096
+    ws = torch.full((ws_bytes // 4 + 4,), float("nan"), device=dev)
+    for dt in (torch.float32, torch.bfloat16):
+        buf = torch.full((m * n + 8,), float("nan"), dtype=dt, device=dev)
+        _hip.check(lib.ferrite_internal_matmul_ragged(xs.data_ptr(), ys.data_ptr(), buf.data_ptr(), m, n, k, 0, int(y_t),
+                                                      _hip.dtype_code(dt), ws.data_ptr(), ws_bytes, st), "matmul")
+        got = to_np(buf[: m * n]).astype(np.float64).reshape(m, n)
+        assert np.all(np.abs(got - exact) <= bound + (bf16_ulp(exact) if dt == torch.bfloat16 else 0.0))
+        assert torch.isnan(buf[m * n :]).all()
+    if not y_t:
+        w = ys.float() * (1 + 2.0**-12)  # rounds back to ys (ties excluded: half an ulp is 2^-9 at least)
+        assert torch.equal(w.bfloat16(), ys)
+        o = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+        u, o2 = torch.empty_like(o), torch.empty_like(o)
+        _hip.check(lib.ferrite_internal_linear_f32w(xs.data_ptr(), w.data_ptr(), o.data_ptr(), None, m, n, k,
+                                                    ws.data_ptr(), ws_bytes, st), "linear")
+        _hip.check(lib.ferrite_internal_linear_f32w(xs.data_ptr(), w.data_ptr(), o2.data_ptr(), u.data_ptr(), m, n, k,
+                                                    ws.data_ptr(), ws_bytes, st), "linear")
+        assert torch.equal(o.view(-1), buf[: m * n]) and torch.equal(u, o)
+        gelu = torch.nn.functional.gelu(u.double(), approximate="tanh")
+        assert ((o2.double() - gelu).abs() <= 2.0**-8 * gelu.abs() + 1e-5).all()
