@@ -1,9 +1,10 @@
-"""Build libferrite_hip.so (the C ABI of include/ferrite_hip.h) for gfx950.
+"""Build libferrite_hip.so (the C ABI of include/ferrite_hip.h) for gfx950, and
+the host module _native.so (csrc/native.cpp, the autograd functions) over it.
 
 Each csrc/*.hip file is compiled by hipcc in parallel and the objects are linked
-into ferrite/libferrite_hip.so, next to the Python package that loads it. The
-library is built in-tree so that it travels with the source tree; nothing is
-installed.
+into ferrite/libferrite_hip.so, next to the Python package that loads it;
+native.cpp is compiled by g++ against torch's headers. Both are built in-tree so
+that they travel with the source tree; nothing is installed.
 
     python ferrite-tpu_amd/build_lib.py [--verbose] [--save-temps DIR]
 """
@@ -16,11 +17,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 OUT = os.path.join(HERE, "ferrite", "libferrite_hip.so")
+NATIVE_OUT = os.path.join(HERE, "ferrite", "_native.so")
 ARCH = "gfx950"
 
 # -packed-fp32-ops: keep hipcc from emitting packed f32 VALU ops (v_pk_*_f32).
@@ -91,21 +94,54 @@ def _compile(src: str, verbose: bool, save_temps: str | None) -> str:
     return obj
 
 
-def build(verbose: bool = False, save_temps: str | None = None) -> str:
-    """Compile every csrc/*.hip for gfx950 and link ferrite/libferrite_hip.so. Returns its path."""
-    os.makedirs(BUILD, exist_ok=True)
-    srcs = _sources()
-    workers = min(len(srcs), max(1, min(8, os.cpu_count() or 1)))
-    with cf.ThreadPoolExecutor(workers) as ex:
-        objs = list(ex.map(lambda s: _compile(s, verbose, save_temps), srcs))
-    tmp = OUT + ".tmp"
-    cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
+def _run(cmd: list[str], verbose: bool, what: str) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"link failed:\n{res.stderr}")
+        raise RuntimeError(f"{what} failed:\n{res.stderr}")
+
+
+def _compile_native(verbose: bool) -> str:
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    obj = os.path.join(BUILD, "native.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-DTORCH_EXTENSION_NAME=_native", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I" + sysconfig.get_paths()["include"]]
+    for path in include_paths("cuda"):
+        cmd += ["-isystem", path]
+    _run([*cmd, "-c", os.path.join(CSRC, "native.cpp"), "-o", obj], verbose, "g++ for csrc/native.cpp")
+    return obj
+
+
+def _link_native(obj: str, verbose: bool) -> None:
+    from torch.utils.cpp_extension import library_paths
+
+    # torch's own libraries are loaded already when the module is imported; libferrite_hip.so lies beside it.
+    cmd = ["g++", "-shared", "-o", NATIVE_OUT + ".tmp", obj, "-L" + os.path.dirname(OUT), "-lferrite_hip",
+           "-Wl,-rpath,$ORIGIN", *("-L" + p for p in library_paths("cuda")), "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_python"]
+    _run(cmd, verbose, "link of _native.so")
+    os.replace(NATIVE_OUT + ".tmp", NATIVE_OUT)
+
+
+def build(verbose: bool = False, save_temps: str | None = None) -> str:
+    """Compile every csrc/*.hip for gfx950 and link ferrite/libferrite_hip.so, then ferrite/_native.so over it.
+    Returns the former's path."""
+    os.makedirs(BUILD, exist_ok=True)
+    srcs = _sources()
+    workers = min(len(srcs) + 1, max(1, min(8, os.cpu_count() or 1)))
+    with cf.ThreadPoolExecutor(workers) as ex:
+        native = ex.submit(_compile_native, verbose)
+        objs = list(ex.map(lambda s: _compile(s, verbose, save_temps), srcs))
+        native_obj = native.result()
+    tmp = OUT + ".tmp"
+    _run([_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,-soname,libferrite_hip.so", "-o", tmp, *objs],
+         verbose, "link")
     os.replace(tmp, OUT)
+    _link_native(native_obj, verbose)
     return OUT
 
 

@@ -105,9 +105,10 @@ __device__ __forceinline__ int xcd_block() {  // neighbouring columns on one XCD
 // w [K,N]. C columns per lane: 2 where rows hold whole pairs (N even, w aligned to a pair),
 // else 1. U of a wave's steps of 16 k are loaded together.
 template <typename TW, typename TO, int C, int MB, int EPI, bool AL>
-__global__ __launch_bounds__(64 * kMaxWaves) void skinny_kernel(const bf16* __restrict__ x, const TW* __restrict__ w,
-                                                                TO* __restrict__ out, bf16* __restrict__ aux, int M,
-                                                                int N, int K, int kslice, int64_t slab) {
+__global__ __launch_bounds__(64 * kMaxWaves) void gemm_skinny_kernel(const bf16* __restrict__ x,
+                                                                     const TW* __restrict__ w, TO* __restrict__ out,
+                                                                     bf16* __restrict__ aux, int M, int N, int K,
+                                                                     int kslice, int64_t slab) {
   extern __shared__ float red[];
   // 128 registers for each of 16 waves
   constexpr int U = C * MB == 1 && AL ? 4 : C * MB < 4 ? 2 : 1;
@@ -183,10 +184,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void skinny_kernel(const bf16* __re
 // product i takes chunk 4 g + i of the step's eight 8-k chunks from both operands, so that
 // a lane's four loads cover 64 consecutive bytes of its row.
 template <typename TO, int MB, int EPI, bool AL>
-__global__ __launch_bounds__(64 * kMaxWaves) void skinny_t_kernel(const bf16* __restrict__ x,
-                                                                  const bf16* __restrict__ w, TO* __restrict__ out,
-                                                                  bf16* __restrict__ aux, int M, int N, int K,
-                                                                  int kslice, int64_t slab) {
+__global__ __launch_bounds__(64 * kMaxWaves) void gemm_skinny_t_kernel(const bf16* __restrict__ x,
+                                                                       const bf16* __restrict__ w,
+                                                                       TO* __restrict__ out, bf16* __restrict__ aux,
+                                                                       int M, int N, int K, int kslice, int64_t slab) {
   extern __shared__ float red[];
   const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
@@ -285,10 +286,10 @@ template <typename TW, typename TO, int EPI, int MB, bool AL>
 int launch(const SkinnyArgs& a, const SkinnyPlan& p, TO* out, hipStream_t stream) {
   const TW* tw = nullptr;
   if constexpr (sizeof(TW) == 2)
-    if (a.w_t) return go(skinny_t_kernel<TO, MB, EPI, AL>, a, p, stream, tw, out);
+    if (a.w_t) return go(gemm_skinny_t_kernel<TO, MB, EPI, AL>, a, p, stream, tw, out);
   if constexpr (AL || MB == 1)
-    if (p.cols == 2) return go(skinny_kernel<TW, TO, 2, MB, EPI, AL>, a, p, stream, tw, out);
-  return go(skinny_kernel<TW, TO, 1, MB, EPI, AL>, a, p, stream, tw, out);
+    if (p.cols == 2) return go(gemm_skinny_kernel<TW, TO, 2, MB, EPI, AL>, a, p, stream, tw, out);
+  return go(gemm_skinny_kernel<TW, TO, 1, MB, EPI, AL>, a, p, stream, tw, out);
 }
 
 template <typename TW, typename TO, int EPI>

@@ -131,6 +131,7 @@ INTERNAL: dict[str, tuple] = {
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+_native = None
 
 
 def lib() -> ctypes.CDLL:
@@ -152,6 +153,27 @@ def lib() -> ctypes.CDLL:
                 fn.argtypes = args
             _lib = handle
     return _lib
+
+
+def native():
+    """Load (once) and return the module of the autograd functions' host side (csrc/native.cpp)."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from ferrite import _native as module
+        except ImportError as e:
+            raise RuntimeError("ferrite/_native.so is missing or does not load: build it with "
+                               "`python ferrite-tpu_amd/build_lib.py` (or __graft_entry__.build()).") from e
+        _native = module
+    return _native
+
+
+def autograd():
+    """:func:`native` for a call that records a custom backward, which no functorch transform can trace."""
+    if torch._C._are_functorch_transforms_active():
+        raise RuntimeError("ferrite's autograd functions have no rule for functorch transforms (vmap, grad, jvp, ...)")
+    return native()
 
 
 def last_error() -> str:

@@ -4,7 +4,7 @@ Reference: src/ferrite/kernels/flash_attention.py. Same public names, arguments,
 defaults and ValueError conditions; the custom VJP wiring of the reference
 (`_flash` with non-differentiable (causal, scale, block_sizes), residuals
 (q, k, v, out, lse), backward = delta + dK/dV kernel + dQ kernel,
-flash_attention.py:315-333) is a torch.autograd.Function here.
+flash_attention.py:315-333) is an autograd function of csrc/native.cpp here.
 
 Kernels (csrc/attention.hip, through include/ferrite_hip.h):
   forward   ferrite_hip_attn_fwd_ex       -> O [B,H,S,D], lse f32 [B,H,S]
@@ -62,47 +62,10 @@ def _on_or_below_diag(qi: int, bq: int, ki: int, bk: int) -> bool:
 # --------------------------------------------------------------------------
 
 
-# Workspaces of the long-context split kernels (partial states and per-pair counts), one per
-# (pass, device, stream, size), zero-filled once: the kernels leave the counts even, as they found
-# them. The forward ("fwd") and the backward's dQ and dK/dV ("bwd", which take turns with one
-# buffer) keep separate ones. A workspace first needed inside a graph capture is allocated there
-# (its zero fill is then part of the graph) and not kept.
-_WORKSPACES: dict[tuple, torch.Tensor] = {}
-
-
-def _workspace(kind: str, nbytes: int, device: torch.device) -> torch.Tensor | None:
-    if nbytes <= 0:
-        return None
-    stream = torch.cuda.current_stream(device)
-    key = (kind, device, stream.cuda_stream, nbytes)
-    ws = _WORKSPACES.get(key)
-    if ws is None:
-        ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
-        if not torch.cuda.is_current_stream_capturing():
-            _WORKSPACES[key] = ws
-    return ws
-
-
-def _ws_args(ws: torch.Tensor | None) -> tuple:
-    return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
-
-
 def _flash_forward(q, k, v, *, causal: bool, scale: float, bs: BlockSizes | None = None):
     """O and the compact logsumexp. Reference: _flash_forward, flash_attention.py:130-175."""
     _hip.require_gpu(q, k, v)
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-    b, h, sq, d = q.shape
-    sk = k.shape[2]
-    out = torch.empty_like(q)
-    lse = torch.empty((b, h, sq), dtype=torch.float32, device=q.device)
-    lib, dt = _hip.lib(), _hip.dtype_code(q.dtype)
-    ws = _workspace("fwd", lib.ferrite_hip_attn_fwd_workspace(b, h, sq, sk, d, dt, int(causal)), q.device)
-    rc = lib.ferrite_hip_attn_fwd_ex(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-        b, h, sq, sk, d, dt, int(causal), float(scale), *_ws_args(ws), _hip.stream_of(q),
-    )
-    _hip.check(rc, "ferrite_flash_attention_fwd")
-    return out, lse
+    return _hip.native().flash_forward(q.contiguous(), k.contiguous(), v.contiguous(), bool(causal), float(scale))
 
 
 def _flash_delta(out, do):
@@ -121,28 +84,7 @@ def _flash_backward_fused(q, k, v, out, do, lse, *, causal: bool, scale: float):
     """dQ, dK, dV with delta (flash_attention.py:328-329) computed inside the dQ kernel from O
     and dO and handed to dK/dV, which therefore runs second: no separate delta pass."""
     _hip.require_gpu(q, k, v, out, do, lse)
-    q, k, v, out, do, lse = (t.contiguous() for t in (q, k, v, out, do, lse))
-    b, h, sq, d = q.shape
-    sk = k.shape[2]
-    dt = _hip.dtype_code(q.dtype)
-    stream = _hip.stream_of(q)
-    dq = torch.empty_like(q)
-    dk = torch.empty_like(k)
-    dv = torch.empty_like(v)
-    delta = torch.empty((b, h, sq), dtype=torch.float32, device=q.device)
-    lib = _hip.lib()
-    wsa = _ws_args(_workspace("bwd", lib.ferrite_hip_attn_bwd_workspace(b, h, sq, sk, d, dt, int(causal)), q.device))
-    rc = lib.ferrite_hip_attn_bwd_dq_delta_ex(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), lse.data_ptr(), delta.data_ptr(),
-        dq.data_ptr(), b, h, sq, sk, d, dt, int(causal), float(scale), *wsa, stream,
-    )
-    _hip.check(rc, "ferrite_flash_attention_bwd_dq")
-    rc = lib.ferrite_hip_attn_bwd_dkv_ex(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), lse.data_ptr(), delta.data_ptr(),
-        dk.data_ptr(), dv.data_ptr(), b, h, sq, sk, d, dt, int(causal), float(scale), *wsa, stream,
-    )
-    _hip.check(rc, "ferrite_flash_attention_bwd_dkv")
-    return dq, dk, dv
+    return _hip.native().flash_backward(*(t.contiguous() for t in (q, k, v, out, do, lse)), bool(causal), float(scale))
 
 
 def _flash_backward(q, k, v, do, lse, delta, *, causal: bool, scale: float, bs: BlockSizes | None = None):
@@ -158,7 +100,9 @@ def _flash_backward(q, k, v, do, lse, delta, *, causal: bool, scale: float, bs: 
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)
     lib = _hip.lib()
-    wsa = _ws_args(_workspace("bwd", lib.ferrite_hip_attn_bwd_workspace(b, h, sq, sk, d, dt, int(causal)), q.device))
+    ws = torch.zeros(max(lib.ferrite_hip_attn_bwd_workspace(b, h, sq, sk, d, dt, int(causal)), 0), dtype=torch.uint8,
+                     device=q.device)  # zero-filled, as the split kernels leave it
+    wsa = (ws.data_ptr(), ws.numel()) if ws.numel() else (None, 0)
     rc = lib.ferrite_hip_attn_bwd_dkv_ex(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), lse.data_ptr(), delta.data_ptr(),
         dk.data_ptr(), dv.data_ptr(), b, h, sq, sk, d, dt, int(causal), float(scale), *wsa, stream,
@@ -175,26 +119,6 @@ def _flash_backward(q, k, v, do, lse, delta, *, causal: bool, scale: float, bs: 
 # --------------------------------------------------------------------------
 # custom VJP and public API
 # --------------------------------------------------------------------------
-
-
-class _Flash(torch.autograd.Function):
-    """`_flash` of the reference (flash_attention.py:315-333): non-differentiable (causal, scale, bs)."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, causal: bool, scale: float, bs: BlockSizes):
-        # The kernels read dense [B, H, S, D]; the dense copies are what the backward re-reads.
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        out, lse = _flash_forward(q, k, v, causal=causal, scale=scale, bs=bs)
-        ctx.save_for_backward(q, k, v, out, lse)
-        ctx.causal, ctx.scale, ctx.bs = causal, scale, bs
-        return out
-
-    @staticmethod
-    def backward(ctx, do):
-        q, k, v, out, lse = ctx.saved_tensors
-        do = do.to(out.dtype).contiguous()
-        dq, dk, dv = _flash_backward_fused(q, k, v, out, do, lse, causal=ctx.causal, scale=ctx.scale)
-        return dq, dk, dv, None, None, None
 
 
 def _validate(q, k, v, causal, bs):
@@ -229,37 +153,9 @@ def flash_attention(q, k, v, *, causal: bool = True, scale: float | None = None,
     _validate(q, k, v, causal, bs)
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[-1])
-    return _Flash.apply(q, k, v, bool(causal), float(scale), bs)
-
-
-class _FlashQKV(torch.autograd.Function):
-    """Causal attention on the token-major projection [B, S, 3, H, D] -> [B, S, H, D], the
-    head transposes of model/gpt.py:137-138 folded into the kernels' addressing."""
-
-    @staticmethod
-    def forward(ctx, qkv, heads, scale):
-        b, s, three, h, d = qkv.shape
-        o = torch.empty((b, s, h, d), dtype=qkv.dtype, device=qkv.device)
-        lse = torch.empty((b, h, s), dtype=torch.float32, device=qkv.device)
-        rc = _hip.lib().ferrite_hip_attn_fwd_qkv(qkv.data_ptr(), o.data_ptr(), lse.data_ptr(), b, s, h, d,
-                                                 float(scale), _hip.stream_of(qkv))
-        _hip.check(rc, "ferrite_flash_attention_fwd")
-        ctx.save_for_backward(qkv, o, lse)
-        ctx.scale = scale
-        return o
-
-    @staticmethod
-    def backward(ctx, do):
-        qkv, o, lse = ctx.saved_tensors
-        b, s, _, h, d = qkv.shape
-        do = do.to(o.dtype).contiguous()
-        dqkv = torch.empty_like(qkv)
-        delta = torch.empty((b, h, s), dtype=torch.float32, device=qkv.device)
-        rc = _hip.lib().ferrite_hip_attn_bwd_qkv(qkv.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr(),
-                                                 delta.data_ptr(), dqkv.data_ptr(), b, s, h, d, float(ctx.scale),
-                                                 _hip.stream_of(qkv))
-        _hip.check(rc, "ferrite_flash_attention_bwd")
-        return dqkv, None, None
+    _hip.require_gpu(q, k, v)
+    _hip.dtype_code(q.dtype)
+    return _hip.autograd().flash(q, k, v, bool(causal), float(scale))
 
 
 def flash_attention_qkv_supported(qkv, heads: int) -> bool:
@@ -280,12 +176,9 @@ def flash_attention_qkv(qkv, heads: int, *, scale: float | None = None):
     if not flash_attention_qkv_supported(qkv, heads):
         raise ValueError(f"flash_attention_qkv needs bf16 [B, S, 3*H*D] on the GPU with D in (64, 128) and S % 64 == 0; "
                          f"got {tuple(qkv.shape)} {qkv.dtype} for {heads} heads")
-    b, s, c = qkv.shape
-    d = c // (3 * heads)
     if scale is None:
-        scale = 1.0 / math.sqrt(d)
-    o = _FlashQKV.apply(qkv.contiguous().view(b, s, 3, heads, d), heads, float(scale))
-    return o.view(b, s, heads * d)
+        scale = 1.0 / math.sqrt(qkv.shape[-1] // (3 * heads))
+    return _hip.autograd().flash_qkv(qkv, heads, float(scale))
 
 
 def flash_attention_reference(q, k, v, *, causal: bool = True, scale: float | None = None):

@@ -32,7 +32,7 @@ from ferrite import platform
 from ferrite.kernels.flash_attention import (BlockSizes, flash_attention, flash_attention_qkv,
                                             flash_attention_qkv_supported, flash_attention_reference)
 from ferrite.kernels.heads import merge_heads, split_heads
-from ferrite.kernels.matmul import matmul, mlp_gelu
+from ferrite.kernels.matmul import linear, mlp_gelu_rounded
 from ferrite.kernels.rmsnorm import rmsnorm, rmsnorm_reference
 
 ROUTES = ("pallas", "xla")
@@ -163,21 +163,20 @@ def param_count(params) -> int:
 
 def _linear(x, w, cfg: GPTConfig):
     """[..., in] @ [in, out] in cfg.dtype with f32 accumulation (gpt.py:95-104)."""
+    if cfg.linear == "pallas":
+        return linear(x.to(cfg.dtype), w)
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1]).to(cfg.dtype)
     w = w.to(cfg.dtype)
-    if cfg.linear == "pallas":
-        y = matmul(x2, w)
-    else:
-        y = torch.matmul(x2, w)  # f32 accumulation, rounded to cfg.dtype
+    y = torch.matmul(x2, w)  # f32 accumulation, rounded to cfg.dtype
     return y.reshape(*lead, w.shape[1])
 
 
 def _mlp(y, layer, cfg: GPTConfig):
     """gelu(y @ w1) @ w2 (gpt.py:141). The bf16 kernel route fuses the GELU and its derivative
-    into the matmul kernels (mlp_gelu); otherwise two linears around torch's tanh GELU."""
+    into the matmul kernels (mlp_gelu_rounded); otherwise two linears around torch's tanh GELU."""
     if cfg.linear == "pallas" and cfg.dtype == torch.bfloat16:
-        return mlp_gelu(y.to(cfg.dtype), layer["w1"].to(cfg.dtype), layer["w2"].to(cfg.dtype))
+        return mlp_gelu_rounded(y.to(cfg.dtype), layer["w1"], layer["w2"])
     return _linear(F.gelu(_linear(y, layer["w1"], cfg), approximate="tanh"), layer["w2"], cfg)
 
 

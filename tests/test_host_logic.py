@@ -45,3 +45,16 @@ def test_attention_schedules(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, out.stderr[-4000:]
     assert "all checks passed" in out.stdout
+
+
+def test_internal_entry_points_match_their_header():
+    """_hip.INTERNAL binds exactly what csrc/internal_api.h declares, and none of it is in the C ABI."""
+    import os
+    import re
+
+    from ferrite import _hip
+    from tests.conftest import ROOT
+
+    text = open(os.path.join(ROOT, "ferrite-tpu_amd", "csrc", "internal_api.h")).read()
+    declared = set(re.findall(r"^(?:int|int64_t) (ferrite_internal_\w+)\(", text, re.M))
+    assert declared == set(_hip.INTERNAL) and not declared & set(_hip.SIGNATURES)
