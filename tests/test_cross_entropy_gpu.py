@@ -78,3 +78,52 @@ def test_validation(dev):
         cross_entropy_rows(torch.zeros(4, 8, device=dev, dtype=torch.bfloat16), torch.zeros(4, dtype=torch.long, device=dev))
     with pytest.raises(ValueError):
         cross_entropy_rows(torch.zeros(4, 8, device=dev), torch.zeros(5, dtype=torch.long, device=dev))
+
+
+@pytest.mark.parametrize("n,v", [
+    (3, 1), (70, 3), (7, 33),            # rows inside one 128-byte line, and just past one
+    (9, 512), (9, 513),                  # one wave per row, then two (backward)
+    (6, 2048), (6, 2049), (5, 5121),     # then four, with whole and ragged batches
+    (3, 50257),
+])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_row_lengths_and_alignment(dev, n, v, shift):
+    """Every split of a row (line-aligned vectors, the elements around them) and an unaligned base,
+    against torch in float64; nothing outside the gradient is written."""
+    x, t = _case(n, v, n * 31 + v)
+    flat = torch.empty(n * v + shift, device=dev)
+    flat[shift:] = torch.from_numpy(x).to(dev).view(-1)
+    xt, tt = flat[shift:].view(n, v), torch.from_numpy(t).to(dev)
+    loss, lse = cross_entropy_rows(xt, tt)
+    x64 = xt.double()
+    ref = torch.logsumexp(x64, 1)
+    # f32 sums of up to 50257 terms by fours, logs of them: 2^-20 relative is four times what is seen
+    assert ((lse.double() - ref).abs() <= 2.0**-20 * ref.abs().clamp(min=1)).all()
+    assert ((loss.double() - (ref - x64[torch.arange(n), tt])).abs() <= 2.0**-20 * x64.abs().max().clamp(min=1)).all()
+    from ferrite import _hip
+
+    p = torch.softmax(x64, 1)
+    p[torch.arange(n), tt] -= 1
+    dloss = torch.ones((), device=dev)
+    for dt, bar in ((torch.float32, 2.0**-18), (torch.bfloat16, 2.0**-8)):
+        buf = torch.full((n * v + shift + 8,), float("nan"), device=dev, dtype=dt)
+        g = buf[shift : shift + n * v]
+        _hip.check(_hip.lib().ferrite_hip_cross_entropy_bwd(xt.data_ptr(), tt.data_ptr(), lse.data_ptr(), dloss.data_ptr(),
+                                                            1.0, g.data_ptr(), n, v, _hip.dtype_code(dt),
+                                                            _hip.stream_of(xt)), "ce_bwd")
+        assert ((g.view(n, v).double() - p).abs() <= bar * p.abs() + 2.0**-20).all()
+        assert torch.isnan(buf[:shift]).all() and torch.isnan(buf[shift + n * v :]).all()
+
+
+@pytest.mark.parametrize("v", [40, 700, 4096])
+def test_infinite_logits(dev, v):
+    """-inf logits (a mask) add nothing, a row with +inf has an infinite logsumexp, as torch's."""
+    x, t = _case(4, v, v)
+    x[0, ::2] = -np.inf
+    x[1, :] = -np.inf
+    x[2, 5] = np.inf
+    x[3, 7] = x[3, v - 1] = np.inf
+    t[:] = 3
+    xt = torch.from_numpy(x).to(dev)
+    _, lse = cross_entropy_rows(xt, torch.from_numpy(t).to(dev))
+    torch.testing.assert_close(lse, torch.logsumexp(xt, 1), rtol=1e-5, atol=0)
