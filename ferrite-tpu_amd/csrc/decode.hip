@@ -19,22 +19,29 @@
 #include <algorithm>
 
 #include "common.h"
+#include "internal_api.h"
 
 namespace ferrite {
 namespace {
 
-constexpr int kDecThreads = 256;  // 4 waves
 constexpr int kUnroll = 4;        // row steps whose loads are issued together
-// Keys per workgroup: the smallest power of two from kChunkMin up that keeps
-// the grid (B H chunks) within kGridTarget workgroups, two per CU of MI355X, so
-// that each wave streams one long contiguous stretch of the cache with kUnroll
-// row steps of non-temporal loads in flight. Measured on MI355X against the
-// previous fixed choice (1024-key chunks for grids of >= 512 such workgroups,
-// else 256; two row steps per batch of loads), one of the B sequences at a
-// third of the cache: 8x32x8192x128 bf16 186.7 -> 162.4 us (4096-key chunks),
-// 32x32x2048x128 bf16 190.9 -> 160.2 us, 8x16x8192x128 f32 168.8 -> 155.3 us,
-// 1x32x8192x128 bf16 28.6 -> 20 us.
-constexpr int kChunkMin = 256;
+// Workgroups per head (chunks): the cache's rows over the smallest power of two from
+// kChunkMin up that keeps the grid (B H chunks) within kGridTarget workgroups, two
+// per CU of MI355X, so that each wave streams one long contiguous stretch of the
+// cache with kUnroll row steps of non-temporal loads in flight. The cache's rows (not a
+// sequence's keys) are cut evenly over the waves of a head's workgroups: cutting the
+// keys evenly instead helps some mixes of lengths and costs others (8x32x8192x128 bf16
+// filled from a third to all of the cache 124 -> 147 us, 32x32x2048x128 136 -> 130).
+// Measured on MI355X, one of the B sequences at a third of the cache: 8x32x8192x128
+// bf16 162.4 us, 32x32x2048x128 bf16 160.2 us, 8x16x8192x128 f32 155.3 us,
+// 1x32x8192x128 bf16 20 us.
+//
+// Grids of few workgroups are bound by latency. Chunks down to 128 keys shorten a wave's
+// chain of loads (3x5x900x256 f32 26.7 -> 17.7 us, 1x1x6590x256 bf16 19.0 -> 17.4 us); where
+// one workgroup of 16 waves reaches the whole cache in two batches of loads a wave, it
+// does, and there is no second pass (8x4x512x128 12.1 -> 9.3 us; with four batches a wave
+// 2x8x2048x64 took 14.7 us, 7.8 in two passes).
+constexpr int kChunkMin = 128;
 constexpr int64_t kGridTarget = 512;
 
 template <typename T>
@@ -78,28 +85,33 @@ __device__ __forceinline__ void merge_state(float& m, float& l, float* acc, floa
   m = mn;
 }
 
-// grid (chunks, H, B), `chunk` keys per workgroup (a power of two >= kChunkMin).
-// Partials: [B, H, chunks, D + 2] = (acc[D], m, l) in the log2 domain.
-template <typename T, int D, bool DIRECT>
-__global__ __launch_bounds__(kDecThreads) void decode_attn_kernel(const T* __restrict__ q, const T* __restrict__ k_new,
+// Rows of a wave's step of loads.
+template <typename T, int D>
+constexpr int kStepRows = 64 / (D / Vec16<T>::N) * kUnroll;
+
+// grid (chunks, H, B); wave_rows (whole steps) rows of the cache per wave. new_stride: elements from one sequence's q, k_new and v_new to the
+// next's. Partials: [B, H, chunks, D + 2] = (acc[D], m, l) in the log2 domain.
+template <typename T, int D, bool DIRECT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void decode_attn_kernel(const T* __restrict__ q, const T* __restrict__ k_new,
                                                                   const T* __restrict__ v_new, T* __restrict__ k_cache,
                                                                   T* __restrict__ v_cache, const int32_t* __restrict__ pos,
                                                                   T* __restrict__ out, float* __restrict__ part,
-                                                                  int max_len, float c, int chunk) {
+                                                                  int max_len, float c, int64_t new_stride, int wave_rows) {
   constexpr int V = Vec16<T>::N;
   constexpr int LPR = D / V;          // lanes per key row
   constexpr int RPW = 64 / LPR;       // rows per wave step
   static_assert(D % V == 0 && LPR >= 1 && LPR <= 64 && (64 % LPR) == 0, "head dim");
-  // A wave's rows (chunk / 4, a power of two >= kChunkMin / 4) in whole unrolled steps.
-  static_assert((kChunkMin / (kDecThreads / 64)) % (RPW * kUnroll) == 0, "a wave's rows in whole unrolled steps");
-  const int wave_rows = chunk / (kDecThreads / 64);
-  __shared__ float red[kDecThreads / 64][D + 2];
+  __shared__ float red[WAVES][D + 2];
 
   const int h = blockIdx.y, b = blockIdx.z;
   const int H = gridDim.y, nchunks = gridDim.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int grp = lane / LPR, sub = lane % LPR;  // row group within the wave, lane within the row
   const int64_t bh = (int64_t)b * H + h;
+  const int64_t new_row = b * new_stride + (int64_t)h * D;
+  q += new_row;
+  k_new += new_row;
+  v_new += new_row;
   const int p = pos[b];
   const bool valid = p >= 0 && p < max_len;
 
@@ -107,20 +119,20 @@ __global__ __launch_bounds__(kDecThreads) void decode_attn_kernel(const T* __res
   if (valid && blockIdx.x == 0 && wave == 0) {
     for (int e = lane * V; e < D; e += 64 * V) {
       *reinterpret_cast<u32x4*>(k_cache + (bh * max_len + p) * D + e) =
-          *reinterpret_cast<const u32x4*>(k_new + bh * D + e);
+          *reinterpret_cast<const u32x4*>(k_new + e);
       *reinterpret_cast<u32x4*>(v_cache + (bh * max_len + p) * D + e) =
-          *reinterpret_cast<const u32x4*>(v_new + bh * D + e);
+          *reinterpret_cast<const u32x4*>(v_new + e);
     }
   }
 
   float qv[V];
-  load_vec(q + bh * D + sub * V, qv);
+  load_vec(q + sub * V, qv);
   float m = -INFINITY, l = 0.f, acc[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) acc[e] = 0.f;
 
   const int last = valid ? p : -1;  // keys 0..last
-  const int r0 = blockIdx.x * chunk + wave * wave_rows;
+  const int r0 = ((int)blockIdx.x * WAVES + wave) * wave_rows;
   // Rows 0 .. last - 1 of the head's cache through descriptors whose range ends
   // at row `last`: an offset past it reads zeros without touching memory, so
   // the loads need no branch and go out together. Row `last` comes from
@@ -140,8 +152,8 @@ __global__ __launch_bounds__(kDecThreads) void decode_attn_kernel(const T* __res
       __builtin_amdgcn_make_buffer_rsrc(uniform(k_cache + bh * max_len * D), (short)0, (int)cached_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t vrs =
       __builtin_amdgcn_make_buffer_rsrc(uniform(v_cache + bh * max_len * D), (short)0, (int)cached_bytes, 0x00020000);
-  const u32x4 knr = *reinterpret_cast<const u32x4*>(k_new + bh * D + sub * V);
-  const u32x4 vnr = *reinterpret_cast<const u32x4*>(v_new + bh * D + sub * V);
+  const u32x4 knr = *reinterpret_cast<const u32x4*>(k_new + sub * V);
+  const u32x4 vnr = *reinterpret_cast<const u32x4*>(v_new + sub * V);
   for (int rs = 0; rs < wave_rows; rs += RPW * kUnroll) {
     if (r0 + rs > last) break;
     // Raw rows; aux 2 makes the loads non-temporal (the cache is read once a step).
@@ -212,24 +224,26 @@ __global__ __launch_bounds__(kDecThreads) void decode_attn_kernel(const T* __res
     }
   }
   __syncthreads();
-  if (wave != 0 || grp != 0) return;
-  for (int w = 1; w < kDecThreads / 64; ++w) {
-    float a2[V];
+  // A thread per element: the waves' weights 2^(m_w - max), then independent sums over the waves.
+  if (threadIdx.x >= D) return;
+  float mx = -INFINITY;
 #pragma unroll
-    for (int e = 0; e < V; ++e) a2[e] = red[w][sub * V + e];
-    merge_state<V>(m, l, acc, red[w][D], red[w][D + 1], a2);
+  for (int w = 0; w < WAVES; ++w) mx = fmaxf(mx, red[w][D]);
+  float lt = 0.f, at = 0.f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    const float f = mx > -INFINITY ? exp2f(red[w][D] - mx) : 0.f;
+    lt += red[w][D + 1] * f;
+    at += red[w][threadIdx.x] * f;
   }
   if constexpr (DIRECT) {
-    const float inv = valid ? 1.f / l : NAN;
-#pragma unroll
-    for (int e = 0; e < V; ++e) out[bh * D + sub * V + e] = Elem<T>::from_f32(acc[e] * inv);
+    out[bh * D + threadIdx.x] = Elem<T>::from_f32(valid ? at / lt : NAN);
   } else {
     float* dst = part + (bh * nchunks + blockIdx.x) * (D + 2);
-#pragma unroll
-    for (int e = 0; e < V; ++e) dst[sub * V + e] = acc[e];
-    if (sub == 0) {
-      dst[D] = m;
-      dst[D + 1] = l;
+    dst[threadIdx.x] = at;
+    if (threadIdx.x == 0) {
+      dst[D] = mx;
+      dst[D + 1] = lt;
     }
   }
 }
@@ -286,17 +300,21 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float* __rest
   }
 }
 
-int64_t chunk_for(int64_t b, int64_t h, int64_t max_len) {
+int64_t chunks_for(int64_t b, int64_t h, int64_t max_len) {
   int64_t c = kChunkMin;
   while (c < max_len && b * h * cdiv(max_len, c) > kGridTarget) c *= 2;
-  return c;
+  return cdiv(max_len, c);
 }
-int64_t chunks_for(int64_t b, int64_t h, int64_t max_len) { return cdiv(max_len, chunk_for(b, h, max_len)); }
 
 template <typename T, int D>
 int decode_launch(const void* q, const void* kn, const void* vn, void* kc, void* vc, const int32_t* pos, void* out,
-                  int64_t B, int64_t H, int64_t L, float scale, void* ws, int64_t ws_bytes, hipStream_t st) {
-  const int64_t chunk = chunk_for(B, H, L), nch = cdiv(L, chunk);
+                  int64_t B, int64_t H, int64_t L, float scale, void* ws, int64_t ws_bytes, int64_t new_stride,
+                  hipStream_t st) {
+  constexpr int kStep = kStepRows<T, D>;
+  int64_t nch = chunks_for(B, H, L);
+  const bool one_group = nch > 1 && L <= 16 * 2 * kStep;
+  if (one_group) nch = 1;
+  const int wave_rows = (int)(cdiv(cdiv(L, nch * (one_group ? 16 : 4)), (int64_t)kStep) * kStep);
   const float c = scale * kLog2e;
   const dim3 grid((unsigned)nch, (unsigned)H, (unsigned)B);
   auto tq = static_cast<const T*>(q);
@@ -305,16 +323,20 @@ int decode_launch(const void* q, const void* kn, const void* vn, void* kc, void*
   auto ck = static_cast<T*>(kc);
   auto cv = static_cast<T*>(vc);
   auto to = static_cast<T*>(out);
-  if (nch == 1) {
-    hipLaunchKernelGGL((decode_attn_kernel<T, D, true>), grid, dim3(kDecThreads), 0, st, tq, tk, tv, ck, cv, pos, to,
-                       nullptr, (int)L, c, (int)chunk);
+  if (one_group) {
+    hipLaunchKernelGGL((decode_attn_kernel<T, D, true, 16>), grid, dim3(1024), 0, st, tq, tk, tv, ck, cv, pos, to,
+                       nullptr, (int)L, c, new_stride, wave_rows);
+  } else if (nch == 1) {
+    hipLaunchKernelGGL((decode_attn_kernel<T, D, true, 4>), grid, dim3(256), 0, st, tq, tk, tv, ck, cv, pos, to,
+                       nullptr, (int)L, c, new_stride, wave_rows);
   } else {
     if (!ws || ws_bytes < B * H * nch * (D + 2) * (int64_t)sizeof(float))
       return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_decode_attention: workspace too small");
-    hipLaunchKernelGGL((decode_attn_kernel<T, D, false>), grid, dim3(kDecThreads), 0, st, tq, tk, tv, ck, cv, pos, to,
-                       static_cast<float*>(ws), (int)L, c, (int)chunk);
+    hipLaunchKernelGGL((decode_attn_kernel<T, D, false, 4>), grid, dim3(256), 0, st, tq, tk, tv, ck, cv, pos, to,
+                       static_cast<float*>(ws), (int)L, c, new_stride, wave_rows);
     hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)H, (unsigned)B), dim3(std::min(D, 256)), 0, st,
-                       static_cast<const float*>(ws), pos, to, (int)nch, (int)L, (int)chunk);
+                       static_cast<const float*>(ws), pos, to, (int)nch, (int)L,
+                       4 * wave_rows);
   }
   return check_launch("ferrite_decode_attention");
 }
@@ -332,6 +354,14 @@ extern "C" int ferrite_hip_decode_attention(const void* q, const void* k_new, co
                                             void* v_cache, const int32_t* pos, void* out, int64_t b, int64_t h,
                                             int64_t max_len, int64_t d, int dtype, float scale, void* workspace,
                                             int64_t workspace_bytes, void* stream) {
+  return ferrite_internal_decode_attention(q, k_new, v_new, k_cache, v_cache, pos, out, b, h, max_len, d, h * d, dtype,
+                                           scale, workspace, workspace_bytes, stream);
+}
+
+extern "C" int ferrite_internal_decode_attention(const void* q, const void* k_new, const void* v_new, void* k_cache,
+                                                 void* v_cache, const int32_t* pos, void* out, int64_t b, int64_t h,
+                                                 int64_t max_len, int64_t d, int64_t new_stride, int dtype, float scale,
+                                                 void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace ferrite;
   const char* name = "ferrite_hip_decode_attention";
   if (!valid_dtype(dtype)) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": dtype must be FERRITE_F32 or FERRITE_BF16");
@@ -341,12 +371,13 @@ extern "C" int ferrite_hip_decode_attention(const void* q, const void* k_new, co
   if (!q || !k_new || !v_new || !k_cache || !v_cache || !pos || !out)
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": null pointer");
   auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (!a16(q) || !a16(k_new) || !a16(v_new) || !a16(k_cache) || !a16(v_cache) || !a16(out))
+  if (!a16(q) || !a16(k_new) || !a16(v_new) || !a16(k_cache) || !a16(v_cache) || !a16(out) || new_stride < h * d ||
+      new_stride % 8 != 0)
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": tensors must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define FERRITE_DEC_CASE(T, DD)                                                                          \
   if (d == DD) return decode_launch<T, DD>(q, k_new, v_new, k_cache, v_cache, pos, out, b, h, max_len, scale, \
-                                           workspace, workspace_bytes, s)
+                                           workspace, workspace_bytes, new_stride, s)
   if (dtype == FERRITE_BF16) {
     FERRITE_DEC_CASE(bf16, 64);
     FERRITE_DEC_CASE(bf16, 128);

@@ -10,6 +10,7 @@
 // side is read or written in whole contiguous rows and the head-major side in
 // D-element runs, so both sides are coalesced.
 #include "common.h"
+#include "internal_api.h"
 
 namespace ferrite {
 namespace {
@@ -92,6 +93,22 @@ int heads_dispatch(const char* name, void* tok, void* const* heads, int64_t b, i
   return heads_launch<float, SPLIT>(tok, heads, b, s, g, h, d, st);
 }
 
+// A decode step's embedding: one block per row. Four launches of a tensor library (two
+// gathers, the sum, the conversion) cost more than the rest of a short step's layer.
+template <typename TE, typename TO>
+__global__ __launch_bounds__(256) void embed_kernel(const int64_t* __restrict__ tokens, const int32_t* __restrict__ pos,
+                                                    const TE* __restrict__ tok_emb, const TE* __restrict__ pos_emb,
+                                                    TO* __restrict__ out, int64_t dim, int64_t vocab, int64_t seq) {
+  const int64_t r = blockIdx.x;
+  int64_t t = tokens[r], p = pos[r];
+  t += t < 0 ? vocab : 0;
+  p += p < 0 ? seq : 0;
+  if (t < 0 || t >= vocab || p < 0 || p >= seq) __builtin_trap();
+  for (int64_t e = threadIdx.x; e < dim; e += 256)
+    out[r * dim + e] = Elem<TO>::from_f32(Elem<TE>::to_f32(
+        Elem<TE>::from_f32(Elem<TE>::to_f32(tok_emb[t * dim + e]) + Elem<TE>::to_f32(pos_emb[p * dim + e]))));
+}
+
 }  // namespace
 }  // namespace ferrite
 
@@ -104,4 +121,35 @@ extern "C" int ferrite_hip_heads_split(const void* tokens, void* const* heads, i
 extern "C" int ferrite_hip_heads_merge(void* const* heads, void* tokens, int64_t b, int64_t s, int64_t groups,
                                        int64_t h, int64_t d, int dtype, void* stream) {
   return ferrite::heads_dispatch<false>("ferrite_hip_heads_merge", tokens, heads, b, s, groups, h, d, dtype, stream);
+}
+
+extern "C" int ferrite_internal_embed(const int64_t* tokens, const int32_t* pos, const void* tok_emb,
+                                      const void* pos_emb, void* out, int64_t rows, int64_t dim, int64_t vocab,
+                                      int64_t seq, int emb_dtype, int out_dtype, void* stream) {
+  using namespace ferrite;
+  const char* name = "ferrite_internal_embed";
+  if (!valid_dtype(emb_dtype) || !valid_dtype(out_dtype))
+    return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": dtype must be FERRITE_F32 or FERRITE_BF16");
+  if (rows < 0 || rows > 0x7fffffff || dim < 1 || vocab < 1 || seq < 1)
+    return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": sizes out of range");
+  if (rows == 0) return FERRITE_OK;
+  if (!tokens || !pos || !tok_emb || !pos_emb || !out)
+    return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": null pointer");
+  auto go = [&](auto* te, auto* to) {
+    typedef std::remove_const_t<std::remove_pointer_t<decltype(te)>> TE;
+    typedef std::remove_pointer_t<decltype(to)> TO;
+    hipLaunchKernelGGL((embed_kernel<TE, TO>), dim3((unsigned)rows), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       tokens, pos, te, static_cast<const TE*>(pos_emb), to, dim, vocab, seq);
+  };
+  auto to = [&](auto* te) {
+    if (out_dtype == FERRITE_BF16)
+      go(te, static_cast<bf16*>(out));
+    else
+      go(te, static_cast<float*>(out));
+  };
+  if (emb_dtype == FERRITE_BF16)
+    to(static_cast<const bf16*>(tok_emb));
+  else
+    to(static_cast<const float*>(tok_emb));
+  return check_launch(name);
 }

@@ -1292,20 +1292,23 @@ extern "C" int ferrite_internal_matmul_ragged(const void* x, const void* y, void
 }
 
 extern "C" int64_t ferrite_internal_linear_f32w_workspace(const void* x, const float* w, int64_t m, int64_t n,
-                                                          int64_t k) {
+                                                          int64_t k, int w_t) {
   using namespace ferrite;
   if (k < 1 || n < 1 || !skinny_ok(m, n, k)) return -1;
-  return skinny_workspace({x, w, nullptr, nullptr, m, n, k, false, FERRITE_F32, FERRITE_BF16, kEpiNone, nullptr, 0});
+  return skinny_workspace({x, w, nullptr, nullptr, m, n, k, w_t != 0, FERRITE_F32, FERRITE_BF16, kEpiNone, nullptr, 0});
 }
 
 extern "C" int ferrite_internal_linear_f32w(const void* x, const float* w, void* out, void* aux, int64_t m, int64_t n,
-                                            int64_t k, void* workspace, int64_t workspace_bytes, void* stream) {
+                                            int64_t k, int w_t, int out_dtype, void* workspace,
+                                            int64_t workspace_bytes, void* stream) {
   using namespace ferrite;
   const char* name = "ferrite_internal_linear_f32w";
+  if (!valid_dtype(out_dtype) || (aux && (w_t || out_dtype != FERRITE_BF16)))
+    return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": dtype or epilogue not supported");
   if (k < 1 || n < 1 || !skinny_ok(m, n, k))
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": sizes out of range");
   if (!x || !w || !out) return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": null pointer");
-  return skinny_launch({x, w, out, aux, m, n, k, false, FERRITE_F32, FERRITE_BF16, aux ? kEpiGelu : kEpiNone, workspace,
+  return skinny_launch({x, w, out, aux, m, n, k, w_t != 0, FERRITE_F32, out_dtype, aux ? kEpiGelu : kEpiNone, workspace,
                         workspace_bytes},
                        static_cast<hipStream_t>(stream));
 }

@@ -351,9 +351,9 @@ Tensor linear_f32w(const Tensor& x0, const Tensor& w0, const Tensor& aux) {
   const int64_t m = rows_of(x), k = w.size(0), n = w.size(1);
   Tensor out = at::empty(with_last(x, n), x.options());
   if (m == 0 || n == 0) return out;
-  const Tensor ws = bytes_on(ferrite_internal_linear_f32w_workspace(ptr(x), (const float*)ptr(w), m, n, k), x);
-  check(ferrite_internal_linear_f32w(ptr(x), (const float*)ptr(w), ptr(out), ptr(aux), m, n, k, ptr(ws), size_of(ws),
-                                     stream_of(x)),
+  const Tensor ws = bytes_on(ferrite_internal_linear_f32w_workspace(ptr(x), (const float*)ptr(w), m, n, k, 0), x);
+  check(ferrite_internal_linear_f32w(ptr(x), (const float*)ptr(w), ptr(out), ptr(aux), m, n, k, 0, code(x), ptr(ws),
+                                     size_of(ws), stream_of(x)),
         "ferrite_matmul");
   return out;
 }
@@ -422,6 +422,60 @@ Tensor mm_2d(const Tensor& x, const Tensor& y, int64_t m, int64_t n, int64_t k, 
 }
 
 // ---------------------------------------------------------------------------
+// Decode step
+// ---------------------------------------------------------------------------
+// The tied head's f32 logits y @ emb^T of up to 64 rows of bf16 y, emb [V, d] rounded to bf16.
+Tensor tied_logits(const Tensor& y0, const Tensor& emb0) {
+  const Tensor y = y0.contiguous(), emb = emb0.contiguous();
+  const int64_t m = y.size(0), k = y.size(1), n = emb.size(0);
+  Tensor out = at::empty({m, n}, y.options().dtype(at::kFloat));
+  if (emb.scalar_type() != at::kFloat) return mm(y, emb, m, n, k, false, true, at::kFloat, {m, n});
+  const Tensor ws = bytes_on(ferrite_internal_linear_f32w_workspace(ptr(y), (const float*)ptr(emb), m, n, k, 1), y);
+  check(ferrite_internal_linear_f32w(ptr(y), (const float*)ptr(emb), ptr(out), nullptr, m, n, k, 1, FERRITE_F32, ptr(ws),
+                                     size_of(ws), stream_of(y)),
+        "ferrite_matmul");
+  return out;
+}
+
+Tensor embed(const Tensor& tokens0, const Tensor& pos0, const Tensor& tok0, const Tensor& pe0, at::ScalarType dtype) {
+  const Tensor tokens = tokens0.to(at::kLong).contiguous(), pos = pos0.to(at::kInt).contiguous();
+  const Tensor tok = tok0.contiguous(), pe = pe0.contiguous();
+  Tensor out = at::empty({tokens.numel(), tok.size(1)}, tok.options().dtype(dtype));
+  check(ferrite_internal_embed((const int64_t*)ptr(tokens), (const int32_t*)ptr(pos), ptr(tok), ptr(pe), ptr(out),
+                               tokens.numel(), tok.size(1), tok.size(0), pe.size(0), code(tok), code(dtype),
+                               stream_of(tok)),
+        "ferrite_embed");
+  return out;
+}
+
+// q, k_new, v_new [B, H, D] are read as they lie when they share one stride per sequence and their
+// heads are dense (the thirds of a fused projection), else from dense copies.
+Tensor decode_attention(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& kc, const Tensor& vc,
+                        const Tensor& pos0, double scale) {
+  const int64_t b = q0.size(0), h = q0.size(1), d = q0.size(2), max_len = kc.size(2);
+  auto lies = [&](const Tensor& t) {
+    return t.stride(2) == 1 && (h == 1 || t.stride(1) == d) && (b == 1 || t.stride(0) == q0.stride(0)) &&
+           (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+  };
+  int64_t stride = b == 1 ? h * d : q0.stride(0);
+  Tensor q = q0, k = k0, v = v0;
+  if (!(stride >= h * d && stride % 8 == 0 && lies(q) && lies(k) && lies(v))) {
+    q = q.contiguous();
+    k = k.contiguous();
+    v = v.contiguous();
+    stride = h * d;
+  }
+  const Tensor pos = pos0.to(at::kInt).contiguous();
+  Tensor out = at::empty({b, h, d}, q.options());
+  const Tensor ws = bytes_on(ferrite_hip_decode_attention_workspace(b, h, max_len, d), q);
+  check(ferrite_internal_decode_attention(ptr(q), ptr(k), ptr(v), ptr(kc), ptr(vc), (const int32_t*)ptr(pos), ptr(out), b,
+                                          h, max_len, d, stride, code(q), (float)scale, ptr(ws), size_of(ws),
+                                          stream_of(q)),
+        "ferrite_decode_attention");
+  return out;
+}
+
+// ---------------------------------------------------------------------------
 // Softmax cross-entropy
 // ---------------------------------------------------------------------------
 std::tuple<Tensor, Tensor> cross_entropy_rows(const Tensor& logits0, const Tensor& targets0) {
@@ -471,6 +525,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear", &linear, nogil());
   m.def("mlp", &mlp, nogil());
   m.def("mm", &mm_2d, nogil());
+  m.def("tied_logits", &tied_logits, nogil());
+  m.def("embed", &embed, nogil());
+  m.def("decode_attention", &decode_attention, nogil());
   m.def("cross_entropy", &cross_entropy, nogil());
   m.def("cross_entropy_rows", &cross_entropy_rows, nogil());
   m.def("cross_entropy_grad", &cross_entropy_grad, nogil());

@@ -8,9 +8,10 @@ namespace ferrite {
 // Rows up to which the skinny kernels take a product: two 32-row MFMA blocks.
 constexpr int64_t kSkinnyRows = 64;
 
-// x bf16 [M,K]; w [K,N] (or, w_t, [N,K]) bf16, or float [K,N] whose elements are rounded to
-// bf16 as they are read; out f32 or bf16 by out_dtype. epi: kEpiNone, kEpiGelu or
-// kEpiGeluGrad (gelu.h) with a bf16 out and aux. Any sizes and element-aligned pointers.
+// x bf16 [M,K]; w [K,N] (or, w_t, [N,K]) bf16, or float whose elements are rounded to bf16 as
+// they are read; out f32 or bf16 by out_dtype. epi: kEpiNone, kEpiGelu (a float w: not
+// transposed) or kEpiGeluGrad (bf16 w) of gelu.h with a bf16 out and aux. Any sizes and
+// element-aligned pointers.
 struct SkinnyArgs {
   const void* x;
   const void* w;

@@ -180,14 +180,35 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemm_skinny_kernel(const bf16*
   reduce_store<TO, C, MB, EPI>(acc, red, out, aux, M, N, n0, waves);
 }
 
+// The 8 elements of a float w row from k0 + k, rounded to bf16.
+template <bool AL>
+__device__ __forceinline__ u32x4 load_f32w(__amdgpu_buffer_rsrc_t r, uint32_t row_off, int k, int rem) {
+  f32x8 v;
+  if constexpr (AL) {
+    const uint32_t at = k < rem ? row_off + 4 * k : kOut;  // + 16 stays past the range
+    const f32x4 a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, 0, 0));
+    const f32x4 b = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(at + 16), 0, 0));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = a[e];
+      v[4 + e] = b[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)(k + e < rem ? row_off + 4 * (k + e) : kOut), 0, 0));
+  }
+  return u32x4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+}
+
 // w given transposed, [N,K]: a lane's 8 k lie together. 64 k per step in four products:
 // product i takes chunk 4 g + i of the step's eight 8-k chunks from both operands, so that
-// a lane's four loads cover 64 consecutive bytes of its row.
-template <typename TO, int MB, int EPI, bool AL>
+// a lane's four loads cover 64 consecutive bytes of its row (128 of a float w's).
+template <typename TW, typename TO, int MB, int EPI, bool AL>
 __global__ __launch_bounds__(64 * kMaxWaves) void gemm_skinny_t_kernel(const bf16* __restrict__ x,
-                                                                       const bf16* __restrict__ w,
-                                                                       TO* __restrict__ out, bf16* __restrict__ aux,
-                                                                       int M, int N, int K, int kslice, int64_t slab) {
+                                                                       const TW* __restrict__ w, TO* __restrict__ out,
+                                                                       bf16* __restrict__ aux, int M, int N, int K,
+                                                                       int kslice, int64_t slab) {
   extern __shared__ float red[];
   const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
@@ -195,7 +216,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemm_skinny_t_kernel(const bf1
   const int sbeg = (int)blockIdx.y * (kslice / 64), steps = min((K + 63) / 64, sbeg + kslice / 64);
   out += blockIdx.y * slab;
   const bool in = n0 + l32 < N;
-  const uint32_t woff = (uint32_t)((int64_t)l32 * K * 2);
+  const uint32_t woff = (uint32_t)((int64_t)l32 * K * sizeof(TW));
   uint32_t xoff[MB];
 #pragma unroll
   for (int b = 0; b < MB; ++b) xoff[b] = l32 + 32 * b < M ? (uint32_t)((int64_t)(l32 + 32 * b) * K * 2) : kOut;
@@ -206,17 +227,20 @@ __global__ __launch_bounds__(64 * kMaxWaves) void gemm_skinny_t_kernel(const bf1
     for (int r = 0; r < 16; ++r) acc[0][b][r] = 0.f;
   for (int s = sbeg + wave; s < steps; s += waves) {
     const int k0 = s * 64, rem = K - k0;
-    const __amdgpu_buffer_rsrc_t wr = rsrc_of(w + (int64_t)n0 * K + k0, ((int64_t)min(N - n0, 32) * K - k0) * 2);
+    const __amdgpu_buffer_rsrc_t wr = rsrc_of(w + (int64_t)n0 * K + k0, ((int64_t)min(N - n0, 32) * K - k0) * (int64_t)sizeof(TW));
     const __amdgpu_buffer_rsrc_t xrs = rsrc_of(x + k0, ((int64_t)M * K - k0) * 2);
     // The chunks loaded together: all, or fewer where a chunk takes eight element loads.
-    constexpr int F = AL ? 4 : MB == 1 ? 2 : 1;
+    constexpr int F = AL ? (sizeof(TW) == 4 ? 2 : 4) : MB == 1 && sizeof(TW) == 2 ? 2 : 1;
 #pragma clang loop unroll(disable)
     for (int i0 = 0; i0 < 4; i0 += F) {
       u32x4 wv[F], xv[F][MB];
 #pragma unroll
       for (int i = 0; i < F; ++i) {
         const int k = (4 * g + i0 + i) * 8;
-        wv[i] = load_x<AL>(wr, woff, k, in ? rem : 0);
+        if constexpr (sizeof(TW) == 4)
+          wv[i] = load_f32w<AL>(wr, woff, k, in ? rem : 0);
+        else
+          wv[i] = load_x<AL>(wr, woff, k, in ? rem : 0);
 #pragma unroll
         for (int b = 0; b < MB; ++b) xv[i][b] = load_x<AL>(xrs, xoff[b], k, xoff[b] == kOut ? 0 : rem);
       }
@@ -285,8 +309,8 @@ int go(Kern kern, const SkinnyArgs& a, const SkinnyPlan& p, hipStream_t stream, 
 template <typename TW, typename TO, int EPI, int MB, bool AL>
 int launch(const SkinnyArgs& a, const SkinnyPlan& p, TO* out, hipStream_t stream) {
   const TW* tw = nullptr;
-  if constexpr (sizeof(TW) == 2)
-    if (a.w_t) return go(gemm_skinny_t_kernel<TO, MB, EPI, AL>, a, p, stream, tw, out);
+  if constexpr (sizeof(TW) == 2 || EPI == kEpiNone)
+    if (a.w_t) return go(gemm_skinny_t_kernel<TW, TO, MB, EPI, AL>, a, p, stream, tw, out);
   if constexpr (AL || MB == 1)
     if (p.cols == 2) return go(gemm_skinny_kernel<TW, TO, 2, MB, EPI, AL>, a, p, stream, tw, out);
   return go(gemm_skinny_kernel<TW, TO, 1, MB, EPI, AL>, a, p, stream, tw, out);

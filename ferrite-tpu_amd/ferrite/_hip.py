@@ -125,8 +125,19 @@ INTERNAL: dict[str, tuple] = {
         _c_int,
         [_vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _vp, _c_i64, _vp],
     ),
-    "ferrite_internal_linear_f32w_workspace": (_c_i64, [_vp, _vp, _c_i64, _c_i64, _c_i64]),
-    "ferrite_internal_linear_f32w": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp, _c_i64, _vp]),
+    "ferrite_internal_linear_f32w_workspace": (_c_i64, [_vp, _vp, _c_i64, _c_i64, _c_i64, _c_int]),
+    "ferrite_internal_linear_f32w": (
+        _c_int,
+        [_vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _vp, _c_i64, _vp],
+    ),
+    "ferrite_internal_decode_attention": (
+        _c_int,
+        [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_f32, _vp, _c_i64, _vp],
+    ),
+    "ferrite_internal_embed": (
+        _c_int,
+        [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _vp],
+    ),
 }
 
 _lock = threading.Lock()

@@ -4,8 +4,8 @@ Reference: src/ferrite/serving/engine.py:89-104 (_cache_attention, _write_cache)
 which the reference leaves to XLA; a decode-attention kernel is its own named
 next step. One call (csrc/decode.hip: ferrite_hip_decode_attention) writes the
 new key/value rows into the cache at each sequence's position and attends the
-query over keys 0..pos, split over key chunks (a power of two from 256 keys up,
-as few as keep the grid within 512 workgroups) merged in f32.
+query over keys 0..pos, cut evenly over the waves of one or more workgroups per
+head (as many as keep the grid within 512) and merged in f32.
 """
 
 from __future__ import annotations
@@ -33,22 +33,9 @@ def decode_attention(q, k_new, v_new, k_cache, v_cache, pos, *, scale: float | N
     if pos.shape != (b,):
         raise ValueError("pos must be [B]")
     _hip.require_gpu(q, k_new, v_new, k_cache, v_cache, pos)
-    q, k_new, v_new = q.contiguous(), k_new.contiguous(), v_new.contiguous()
-    pos = pos.to(torch.int32).contiguous()
     if scale is None:
         scale = 1.0 / math.sqrt(d)
-    max_len = k_cache.shape[2]
-    out = torch.empty_like(q)
-    lib = _hip.lib()
-    ws_bytes = lib.ferrite_hip_decode_attention_workspace(b, h, max_len, d)
-    ws = torch.empty(((ws_bytes + 3) // 4,), dtype=torch.float32, device=q.device) if ws_bytes > 0 else None
-    rc = lib.ferrite_hip_decode_attention(
-        q.data_ptr(), k_new.data_ptr(), v_new.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), pos.data_ptr(),
-        out.data_ptr(), b, h, max_len, d, _hip.dtype_code(q.dtype), float(scale), _hip.ptr(ws), max(ws_bytes, 0),
-        _hip.stream_of(q),
-    )
-    _hip.check(rc, "ferrite_decode_attention")
-    return out
+    return _hip.native().decode_attention(q, k_new, v_new, k_cache, v_cache, pos, float(scale))
 
 
 def decode_attention_reference(q, k_new, v_new, k_cache, v_cache, pos, *, scale: float | None = None):

@@ -29,6 +29,7 @@ from typing import Any
 import numpy as np
 import torch
 
+from ferrite import _hip
 from ferrite.graphs import capture_window
 from ferrite.model.gpt import GPTConfig, _attention, _dot_f32, _linear, _merge_heads, _mlp, _norm, _split_heads
 
@@ -120,7 +121,11 @@ def decode_step(params, token, pos, k_cache, v_cache, cfg: GPTConfig):
     (engine.py:107-131). With ``cfg.attention == "pallas"`` the HIP decode-attention kernel does
     the cache write and the attention; otherwise torch restates the reference's XLA math."""
     b = token.shape[0]
-    h = (params["tok_emb"][token] + params["pos_emb"][pos.long()]).to(cfg.dtype)  # [B, d]
+    kernels = cfg.attention == "pallas"
+    if kernels:
+        h = _embed(params, token, pos, cfg)
+    else:
+        h = (params["tok_emb"][token] + params["pos_emb"][pos.long()]).to(cfg.dtype)  # [B, d]
     scale = 1.0 / math.sqrt(cfg.head_dim)
     pending = None
     for i, layer in enumerate(params["layers"]):
@@ -129,8 +134,8 @@ def decode_step(params, token, pos, k_cache, v_cache, cfg: GPTConfig):
         else:
             h, y = _norm(pending, layer["ln1"], h, cfg)
         qkv = _linear(y, layer["wqkv"], cfg).reshape(b, 3, cfg.n_head, cfg.head_dim)
-        q, k, v = (qkv[:, j].contiguous() for j in range(3))  # [B, H, hd]
-        if cfg.attention == "pallas":
+        q, k, v = qkv.unbind(1)  # [B, H, hd]
+        if kernels:
             from ferrite.kernels.decode_attention import decode_attention
 
             a = decode_attention(q, k, v, k_cache[i], v_cache[i], pos, scale=scale)
@@ -142,7 +147,22 @@ def decode_step(params, token, pos, k_cache, v_cache, cfg: GPTConfig):
         h, y2 = _norm(a, layer["ln2"], h, cfg)
         pending = _mlp(y2, layer, cfg)
     _, y = _norm(pending, params["ln_f"], h, cfg)
+    if kernels and _few_rows_head(y, params["tok_emb"]):
+        return _hip.native().tied_logits(y, params["tok_emb"])
     return _dot_f32(y, params["tok_emb"].to(cfg.dtype).t())
+
+
+def _embed(params, token, pos, cfg: GPTConfig):
+    """The decode step's embeddings [B, d] in cfg.dtype, in one kernel."""
+    _hip.require_gpu(token, pos, params["tok_emb"], params["pos_emb"])
+    return _hip.native().embed(token, pos, params["tok_emb"], params["pos_emb"], cfg.dtype)
+
+
+def _few_rows_head(y, emb) -> bool:
+    """Whether the tied head runs on the few-rows kernel, which reads the embedding as it is: up to
+    64 rows of bf16 and 2^24 weights (beyond those the library product is level or faster)."""
+    return y.dtype == torch.bfloat16 and emb.dtype in (torch.float32, torch.bfloat16) and y.shape[0] <= 64 \
+        and emb.numel() <= 1 << 24
 
 
 # The serving engine: captured prefill per bucket, one captured decode step.

@@ -423,14 +423,19 @@ def test_few_rows(dev, m, n, k, y_t):
         got = to_np(buf[: m * n]).astype(np.float64).reshape(m, n)
         assert np.all(np.abs(got - exact) <= bound + (bf16_ulp(exact) if dt == torch.bfloat16 else 0.0))
         assert torch.isnan(buf[m * n :]).all()
+    w = ys.float() * (1 + 2.0**-12)
+    o32 = torch.empty((m, n), device=dev)
+    _hip.check(lib.ferrite_internal_linear_f32w(xs.data_ptr(), w.data_ptr(), o32.data_ptr(), None, m, n, k, int(y_t),
+                                                _hip.F32, ws.data_ptr(), ws_bytes, st), "linear")
+    assert np.all(np.abs(to_np(o32).astype(np.float64) - exact) <= bound)
     if not y_t:
         w = ys.float() * (1 + 2.0**-12)  # rounds back to ys (ties excluded: half an ulp is 2^-9 at least)
         assert torch.equal(w.bfloat16(), ys)
         o = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
         u, o2 = torch.empty_like(o), torch.empty_like(o)
-        _hip.check(lib.ferrite_internal_linear_f32w(xs.data_ptr(), w.data_ptr(), o.data_ptr(), None, m, n, k,
+        _hip.check(lib.ferrite_internal_linear_f32w(xs.data_ptr(), w.data_ptr(), o.data_ptr(), None, m, n, k, 0, _hip.BF16,
                                                     ws.data_ptr(), ws_bytes, st), "linear")
-        _hip.check(lib.ferrite_internal_linear_f32w(xs.data_ptr(), w.data_ptr(), o2.data_ptr(), u.data_ptr(), m, n, k,
+        _hip.check(lib.ferrite_internal_linear_f32w(xs.data_ptr(), w.data_ptr(), o2.data_ptr(), u.data_ptr(), m, n, k, 0, _hip.BF16,
                                                     ws.data_ptr(), ws_bytes, st), "linear")
         assert torch.equal(o.view(-1), buf[: m * n]) and torch.equal(u, o)
         gelu = torch.nn.functional.gelu(u.double(), approximate="tanh")

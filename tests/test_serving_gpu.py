@@ -169,3 +169,50 @@ def test_engine_close_releases_graphs(dev):
     with Engine(params, cfg, ServeConfig(batch=2, max_len=128, buckets=(32,))) as eng2:
         got, _ = eng2.generate([[1, 2, 3], [4, 5]], 6)
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("b,h,L,d,dtype", [
+    (3, 2, 512, 128, torch.bfloat16),   # one workgroup of 16 waves per head
+    (2, 3, 513, 128, torch.bfloat16),   # one row more: chunks and a second pass
+    (1, 2, 128, 64, torch.bfloat16),    # one workgroup of 4 waves
+    (2, 1, 130, 256, torch.float32),
+    (24, 22, 300, 64, torch.bfloat16),  # many heads: one workgroup of 4 waves, rows not a power of two
+])
+def test_decode_attention_reads_a_projection_in_place(dev, b, h, L, d, dtype):
+    """q, k and v as thirds of one [B, 3, H, D] projection give bitwise what dense copies do, and both
+    match the torch restatement (f32 sums in another order; one bf16 rounding of the output)."""
+    g = torch.Generator(device=dev).manual_seed(b * L)
+    qkv = torch.randn(b, 3, h, d, device=dev, generator=g).to(dtype)
+    pos = torch.randint(0, L, (b,), device=dev, generator=g, dtype=torch.int32)
+    pos[0] = L - 1
+    caches = [torch.randn(b, h, L, d, device=dev, generator=g).to(dtype) for _ in range(2)]
+    outs = []
+    for dense in (False, True):
+        kc, vc = (c.clone() for c in caches)
+        q, k, v = (t.contiguous() if dense else t for t in qkv.unbind(1))
+        outs.append((decode_attention(q, k, v, kc, vc, pos), kc, vc))
+    assert all(torch.equal(a, c) for a, c in zip(*outs))
+    kc, vc = (c.clone() for c in caches)
+    ref = decode_attention_reference(*qkv.unbind(1), kc, vc, pos)
+    assert torch.equal(kc, outs[0][1]) and torch.equal(vc, outs[0][2])
+    bar = 2.0**-7 if dtype == torch.bfloat16 else 1e-5
+    assert ((outs[0][0].float() - ref.float()).abs() <= bar * ref.float().abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("edt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 520])
+def test_decode_embedding_and_head(dev, edt, d):
+    """The decode step's one-kernel embedding is bitwise the gathers, sum and cast, negative indices
+    included, and the few-rows head is the rounded embedding's product to f32 sums."""
+    from ferrite import _hip
+
+    g = torch.Generator(device=dev).manual_seed(d)
+    tok, pe = (torch.randn(n, d, device=dev, generator=g).to(edt) for n in (300, 70))
+    t = torch.tensor([0, 299, -1, 17], device=dev)
+    p = torch.tensor([69, 0, 3, -70], dtype=torch.int32, device=dev)
+    for dt in (torch.bfloat16, torch.float32):
+        assert torch.equal(_hip.native().embed(t, p, tok, pe, dt), (tok[t] + pe[p.long()]).to(dt))
+    y = torch.randn(5, d, device=dev, generator=g).bfloat16()
+    ref = y.double() @ tok.bfloat16().double().t()
+    bound = 2.0**-20 * (y.double().abs() @ tok.bfloat16().double().abs().t())
+    assert ((_hip.native().tied_logits(y, tok).double() - ref).abs() <= bound).all()
