@@ -203,7 +203,187 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const TX* __restrict_
   }
 }
 
-// General path: any dim and alignment. Two sweeps over the row; the second
+// ---------------------------------------------------------------------------
+// Rows the fast path does not take (dim % 8 != 0, unaligned, or wider than 4096): a group of
+// G threads (a wave, a workgroup of 4 waves, or one of 16) owns a row and keeps it in
+// registers, up to VPL units of CW elements per thread, unit t + G i for thread t: CW = 8 where
+// rows hold whole aligned eights, 2 where they hold aligned pairs, else single elements. The
+// row is read once and all of its loads go out together. us on one MI355X, the two-sweep
+// kernels below (one wave per row) / these, add+norm and backward:
+//   9660 x 5504 f32   292 / 182 (4.7 TB/s)   388 / 172     8192 x 8192 bf16  187 / 95    254 / 113
+//   512 x 8192 f32     78 / 16                94 / 27      27013 x 915 f32   107 / 94    134 / 77
+//   50000 x 1110 bf16 148 / 112              221 / 166     60000 x 77 bf16    19 / 14     60 / 42
+// Single bf16 elements are bound by the CU's address path, which takes an element load as long
+// as one of 16 bytes, and by registers; there the two sweeps' many light waves stay the
+// better ones between 256 and 4096 columns (27013 x 915: 47 / 52 and 72 / 89, 10376 x 2945:
+// 67 / 72 and 106 / 168), as they do for the plain norm of 1025 to 2048 columns of pairs
+// (50000 x 1110: 69 / 83) and the backward of wider pairs (10376 x 2946: 102 / 104):
+// group_wins and group_wins_bwd.
+// ---------------------------------------------------------------------------
+template <typename T, int CW>
+struct Unit {
+  float v[CW];
+};
+template <typename T, int CW>
+__device__ __forceinline__ void load_unit(const T* p, Unit<T, CW>& u) {
+  if constexpr (CW == 8) {
+    Raw8<T> r;
+    ld8_nt(p, r);
+    unpack8(r, u.v);
+  } else if constexpr (CW == 2 && sizeof(T) == 2) {
+    const uint32_t w = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
+    u.v[0] = __uint_as_float(w << 16);
+    u.v[1] = __uint_as_float(w & 0xffff0000u);
+  } else if constexpr (CW == 2) {
+    const f32x2 w = __builtin_nontemporal_load(reinterpret_cast<const f32x2*>(p));
+    u.v[0] = w[0];
+    u.v[1] = w[1];
+  } else {
+    u.v[0] = Elem<T>::to_f32(*p);
+  }
+}
+template <typename T, int CW>
+__device__ __forceinline__ void store_unit(T* p, const float (&v)[CW]) {
+  if constexpr (CW == 8)
+    st8_nt(p, v);
+  else if constexpr (CW == 2 && sizeof(T) == 2)
+    *reinterpret_cast<uint32_t*>(p) = pack_bf16(v[0], v[1]);
+  else if constexpr (CW == 2)
+    *reinterpret_cast<f32x2*>(p) = f32x2{v[0], v[1]};
+  else
+    *p = Elem<T>::from_f32(v[0]);
+}
+
+// A thread's weights, read once: a load of a single element takes the CU's address path as long as
+// one of 16 bytes, so weights read again for every row would halve the rows' rate.
+template <int CW, int VPL, int G, typename TW>
+__device__ __forceinline__ void load_weights(const TW* w, int dim, int t, float (&wv)[VPL][CW]) {
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const int c = (t + G * i) * CW;
+    if (c < dim) {
+      if constexpr (CW == 8) {
+        load8(w + c, wv[i]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < CW; ++e) wv[i][e] = Elem<TW>::to_f32(w[c + e]);
+      }
+    }
+  }
+}
+
+// Sum over a group of G threads, in every one of its threads (G > 64: the whole workgroup).
+template <int G>
+__device__ __forceinline__ float group_sum(float x, float* lds) {
+  x = wave_sum(x);
+  if constexpr (G > 64) {
+    __syncthreads();  // the previous sum has been read
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = x;
+    __syncthreads();
+    x = 0.f;
+#pragma unroll
+    for (int w = 0; w < G / 64; ++w) x += lds[w];
+  }
+  return x;
+}
+
+template <typename TX, typename TW, bool RES, int CW, int VPL, int G>
+__global__ __launch_bounds__((G < 256 ? 256 : G)) void rmsnorm_group_kernel(
+    const TX* __restrict__ x, const TX* __restrict__ r, const TW* __restrict__ w, TX* __restrict__ h,
+    TX* __restrict__ y, int64_t rows, int dim, float inv_dim, float eps) {
+  constexpr int kRows = G < 256 ? 256 / G : 1;  // rows per workgroup and pass
+  __shared__ float lds[16];
+  const int t = threadIdx.x % G;
+  float wv[VPL][CW];
+  load_weights<CW, VPL, G>(w, dim, t, wv);
+  for (int64_t row0 = (int64_t)blockIdx.x * kRows; row0 < rows; row0 += (int64_t)gridDim.x * kRows) {
+    const int64_t row = row0 + threadIdx.x / G;
+    if (G == 64 && row >= rows) return;
+    const int64_t off = row * dim;
+    Unit<TX, CW> hv[VPL], rv[VPL];
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = (t + G * i) * CW;
+      if (c < dim) {
+        load_unit<TX, CW>(x + off + c, hv[i]);
+        if constexpr (RES) load_unit<TX, CW>(r + off + c, rv[i]);
+      }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = (t + G * i) * CW;
+      if (c < dim) {
+#pragma unroll
+        for (int e = 0; e < CW; ++e) {
+          if constexpr (RES) hv[i].v[e] += rv[i].v[e];
+          ss += hv[i].v[e] * hv[i].v[e];
+        }
+        if constexpr (RES) store_unit<TX, CW>(h + off + c, hv[i].v);
+      }
+    }
+    ss = group_sum<G>(ss, lds);
+    const float inv = __builtin_amdgcn_rsqf(ss * inv_dim + eps);
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = (t + G * i) * CW;
+      if (c < dim) {
+        float yv[CW];
+#pragma unroll
+        for (int e = 0; e < CW; ++e) yv[e] = (hv[i].v[e] * inv) * wv[i][e];
+        store_unit<TX, CW>(y + off + c, yv);
+      }
+    }
+  }
+}
+
+// The unit of such rows, and the smallest group that holds a row: 32 elements a thread in units of
+// 8 or 2, 16 single ones, half of that with 16 waves (128 registers each); 0 where none does.
+int unit_of(int64_t dim, bool a16, bool pairs) {
+  return dim % 8 == 0 && a16 ? 8 : dim % 2 == 0 && pairs ? 2 : 1;
+}
+int group_of(int64_t dim, int unit) {
+  const int64_t per = unit == 1 ? 16 : 32;
+  return dim <= 64 * per ? 64 : dim <= 256 * per ? 256 : dim <= 512 * per ? 1024 : 0;
+}
+bool group_wins(int esize, int unit, int64_t dim, bool residual) {
+  if (esize == 4 || unit == 8 || dim <= 256) return true;
+  return unit == 2 ? residual || dim <= 1024 || dim > 2048 : dim > 4096;
+}
+bool group_wins_bwd(int esize, int unit, int64_t rows, int64_t dim) {
+  if (esize == 4 || unit == 8 || dim <= 256) return true;
+  return unit == 2 ? dim <= 2048 : rows * dim <= (int64_t)1 << 22;
+}
+bool aligned_to(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; }
+
+// Runs the statement with CW, VPL and G as constants.
+#define FERRITE_GROUP_G(CW_, VPL_, g, ...)                       \
+  do {                                                           \
+    constexpr int CW = CW_, VPL = VPL_;                          \
+    if ((g) == 64) {                                             \
+      constexpr int G = 64;                                      \
+      __VA_ARGS__;                                               \
+    } else if ((g) == 256) {                                     \
+      constexpr int G = 256;                                     \
+      __VA_ARGS__;                                               \
+    } else if constexpr (CW_ * VPL_ <= (CW_ == 1 ? 8 : 16)) {    \
+      constexpr int G = 1024;                                    \
+      __VA_ARGS__;                                               \
+    }                                                            \
+  } while (0)
+// Half the units per thread where that reaches the row (fewer registers and predicated loads).
+#define FERRITE_GROUP(unit, g, dim, ...)                                                           \
+  do {                                                                                             \
+    if ((unit) == 8) {                                                                             \
+      if ((dim) <= (g) * 16) FERRITE_GROUP_G(8, 2, g, __VA_ARGS__); else FERRITE_GROUP_G(8, 4, g, __VA_ARGS__); \
+    } else if ((unit) == 2) {                                                                      \
+      if ((dim) <= (g) * 16) FERRITE_GROUP_G(2, 8, g, __VA_ARGS__); else FERRITE_GROUP_G(2, 16, g, __VA_ARGS__); \
+    } else {                                                                                       \
+      if ((dim) <= (g) * 8) FERRITE_GROUP_G(1, 8, g, __VA_ARGS__); else FERRITE_GROUP_G(1, 16, g, __VA_ARGS__); \
+    }                                                                                              \
+  } while (0)
+
+// Rows that no group takes. Two sweeps over the row; the second
 // recomputes h = x + r from the same inputs (bitwise the same f32 values).
 template <typename TX, typename TW, bool RES>
 __global__ __launch_bounds__(256) void rmsnorm_rows_generic_kernel(const TX* __restrict__ x, const TX* __restrict__ r,
@@ -278,6 +458,21 @@ int launch(const void* x, const void* r, const void* w, void* h, void* y, int64_
     else
       FERRITE_RMS_CASE(8, 1);
 #undef FERRITE_RMS_CASE
+    return check_launch(RES ? "ferrite_add_rmsnorm" : "ferrite_rmsnorm");
+  }
+  auto all = [&](int bytes) {
+    return aligned_to(x, bytes) && aligned_to(y, bytes) && (!RES || (aligned_to(r, bytes) && aligned_to(h, bytes)));
+  };
+  const int unit = unit_of(dim, all(16) && aligned_to(w, 16), all(2 * (int)sizeof(TX)));
+  const int group = group_wins((int)sizeof(TX), unit, dim, RES) ? group_of(dim, unit) : 0;
+  if (group) {
+    const int64_t per_block = group < 256 ? 256 / group : 1;
+    // Persistent from eight workgroups of four waves per CU on.
+    const int64_t most = group > 256 ? 512 : 2048;
+    const dim3 ggrid((unsigned)std::min<int64_t>(cdiv(rows, per_block), most)), gblock(group < 256 ? 256 : group);
+    FERRITE_GROUP(unit, group, dim,
+                  hipLaunchKernelGGL((rmsnorm_group_kernel<TX, TW, RES, CW, VPL, G>), ggrid, gblock, 0, stream, xp, rp, wp,
+                                     hp, yp, rows, (int)dim, inv_dim, eps));
   } else {
     hipLaunchKernelGGL((rmsnorm_rows_generic_kernel<TX, TW, RES>), grid, block, 0, stream, xp, rp, wp, hp, yp, rows,
                        dim, inv_dim, eps);
@@ -394,7 +589,91 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_rows_kernel(const TX* __restr
     partial[(int64_t)blockIdx.x * dim + col] = (red[col] + red[dim + col]) + (red[2 * dim + col] + red[3 * dim + col]);
 }
 
-// General row pass (any dim or alignment): one wave per row, two sweeps. The
+// The backward of the rows the fast path does not take, in groups of G threads as
+// rmsnorm_group_kernel: every thread owns the same columns on every row of its group, so dw
+// accumulates in registers and h and dy are read once (the general passes below read both
+// twice more). One partial row per workgroup, its groups combined through LDS.
+template <typename TX, typename TW, typename TO, bool DIRECT, int CW, int VPL, int G>
+__global__ __launch_bounds__((G < 256 ? 256 : G)) void rmsnorm_bwd_group_kernel(
+    const TX* __restrict__ h, const TW* __restrict__ w, const TX* __restrict__ dy, const TX* __restrict__ dd,
+    TO* __restrict__ dh, float* __restrict__ partial, int64_t rows, int dim, float inv_dim, float eps) {
+  constexpr int kRows = G < 256 ? 256 / G : 1;
+  extern __shared__ float red[];  // [kRows][dim] where kRows > 1
+  __shared__ float lds[2][16];
+  const int t = threadIdx.x % G, grp = threadIdx.x / G;
+  float wv[VPL][CW], acc[VPL][CW];
+  load_weights<CW, VPL, G>(w, dim, t, wv);
+#pragma unroll
+  for (int i = 0; i < VPL; ++i)
+#pragma unroll
+    for (int e = 0; e < CW; ++e) acc[i][e] = 0.f;
+  for (int64_t row0 = (int64_t)blockIdx.x * kRows; row0 < rows; row0 += (int64_t)gridDim.x * kRows) {
+    const int64_t row = row0 + grp;
+    if (G == 64 && row >= rows) break;
+    const int64_t off = row * dim;
+    Unit<TX, CW> hv[VPL], gv[VPL], dv[VPL];
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = (t + G * i) * CW;
+      if (c < dim) {
+        load_unit<TX, CW>(h + off + c, hv[i]);
+        load_unit<TX, CW>(dy + off + c, gv[i]);
+        if constexpr (DIRECT) load_unit<TX, CW>(dd + off + c, dv[i]);
+      }
+    }
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = (t + G * i) * CW;
+      if (c < dim) {
+#pragma unroll
+        for (int e = 0; e < CW; ++e) {
+          s1 += hv[i].v[e] * hv[i].v[e];
+          s2 += (gv[i].v[e] * wv[i][e]) * hv[i].v[e];
+        }
+      }
+    }
+    s1 = group_sum<G>(s1, lds[0]);
+    s2 = group_sum<G>(s2, lds[1]);
+    const float inv = __builtin_amdgcn_rsqf(s1 * inv_dim + eps);
+    const float mean = inv * s2 * inv_dim;  // mean(dxhat * xhat)
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = (t + G * i) * CW;
+      if (c < dim) {
+        float out[CW];
+#pragma unroll
+        for (int e = 0; e < CW; ++e) {
+          const float xh = hv[i].v[e] * inv;
+          out[e] = inv * (gv[i].v[e] * wv[i][e] - xh * mean);
+          if constexpr (DIRECT) out[e] += dv[i].v[e];
+          acc[i][e] += gv[i].v[e] * xh;
+        }
+        store_unit<TO, CW>(dh + off + c, out);
+      }
+    }
+  }
+  float* const dst = kRows > 1 ? red + grp * dim : partial + (int64_t)blockIdx.x * dim;
+#pragma unroll
+  for (int i = 0; i < VPL; ++i) {
+    const int c = (t + G * i) * CW;
+    if (c < dim) {
+#pragma unroll
+      for (int e = 0; e < CW; ++e) dst[c + e] = acc[i][e];
+    }
+  }
+  if constexpr (kRows > 1) {
+    __syncthreads();
+    for (int col = threadIdx.x; col < dim; col += blockDim.x) {
+      float s = 0.f;
+#pragma unroll
+      for (int k = 0; k < kRows; ++k) s += red[k * dim + col];
+      partial[(int64_t)blockIdx.x * dim + col] = s;
+    }
+  }
+}
+
+// Rows that no group takes: one wave per row, two sweeps. The
 // per-row inv goes to the workspace for the column pass below.
 template <typename TX, typename TW, typename TO, bool DIRECT>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_rows_generic_kernel(const TX* __restrict__ h,
@@ -472,17 +751,19 @@ __global__ __launch_bounds__(kDwCols* kDwGroups) void rmsnorm_bwd_dw_kernel(cons
 
 // Workspace of the backward: nparts partial rows of dim floats (nparts <= kBwdMaxParts),
 // then, on the general path only, one float per row. The size query of the C ABI
-// returns the bound over every path; bwd_plan gives what one call really uses.
+// returns the bound over every path; bwd_plan gives what a call asks for: the group
+// kernels use no more than the general passes, whose shapes they took over.
 int64_t bwd_workspace_bytes(int64_t rows, int64_t dim) { return ((int64_t)kBwdMaxParts * dim + rows) * 4; }
 
 struct BwdPlan {
-  bool fast;      // the one-pass row kernel (else the general row + column passes)
-  int nparts;     // partial dw rows
+  bool fast;        // the one-pass row kernel
+  int unit, group;  // else the group kernel (group > 0), or the general row + column passes
+  int nparts;       // partial dw rows
   int64_t bytes;  // workspace bytes this call uses
 };
 
 BwdPlan bwd_plan(const void* h, const void* w, const void* dy, const void* dd, const void* dh, int64_t rows,
-                 int64_t dim) {
+                 int64_t dim, int xsize, int osize) {
   auto aligned16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   BwdPlan p{};
   p.fast = dim % kChunk == 0 && dim <= 64 * kChunk * 8 && aligned16(h) && aligned16(dy) && aligned16(w) &&
@@ -494,6 +775,15 @@ BwdPlan bwd_plan(const void* h, const void* w, const void* dy, const void* dd, c
   else
     p.nparts = (int)std::min<int64_t>(rows, kBwdMaxParts);
   p.bytes = ((int64_t)p.nparts * dim + (p.fast || rows <= 0 ? 0 : rows)) * 4;
+  if (!p.fast && rows > 0) {
+    auto all = [&](int n) {
+      return aligned_to(h, n * xsize) && aligned_to(dy, n * xsize) && aligned_to(dh, n * osize) &&
+             (!dd || aligned_to(dd, n * xsize));
+    };
+    p.unit = unit_of(dim, aligned16(w) && aligned16(h) && aligned16(dy) && aligned16(dh) && (!dd || aligned16(dd)), all(2));
+    p.group = group_wins_bwd(xsize, p.unit, rows, dim) ? group_of(dim, p.unit) : 0;
+    if (p.group) p.nparts = (int)std::min<int64_t>(cdiv(rows, (int64_t)(p.group < 256 ? 256 / p.group : 1)), kBwdMaxParts);
+  }
   return p;
 }
 
@@ -507,7 +797,7 @@ int bwd_launch(const void* h, const void* w, const void* dy, const void* dd, voi
   const TW* wp = static_cast<const TW*>(w);
   TO* op = static_cast<TO*>(dh);
   float* partial = static_cast<float*>(ws);
-  const BwdPlan plan = bwd_plan(h, w, dy, DIRECT ? dd : nullptr, dh, rows, dim);
+  const BwdPlan plan = bwd_plan(h, w, dy, DIRECT ? dd : nullptr, dh, rows, dim, (int)sizeof(TX), (int)sizeof(TO));
   const int nparts = plan.nparts;
   if (rows > 0 && plan.fast) {
     const int vpl = (int)cdiv(dim / kChunk, 64);
@@ -524,6 +814,13 @@ int bwd_launch(const void* h, const void* w, const void* dy, const void* dd, voi
     else
       FERRITE_RMS_BWD_CASE(8);
 #undef FERRITE_RMS_BWD_CASE
+  } else if (rows > 0 && plan.group) {
+    const int g = plan.group;
+    const size_t lds = g < 256 ? (size_t)(256 / g) * dim * sizeof(float) : 0;
+    FERRITE_GROUP(plan.unit, g, dim,
+                  hipLaunchKernelGGL((rmsnorm_bwd_group_kernel<TX, TW, TO, DIRECT, CW, VPL, G>), dim3(nparts),
+                                     dim3(g < 256 ? 256 : g), lds, stream, hp, wp, gp, dp, op, partial, rows, (int)dim,
+                                     inv_dim, eps));
   } else if (rows > 0) {
     float* inv_rows = partial + (int64_t)nparts * dim;
     const int64_t blocks = cdiv(rows, kRowsPerBlock);
@@ -687,7 +984,8 @@ int bwd_entry(const char* name, const void* h, const void* weight, const void* d
   if (!weight || !dweight || (!noalloc && !workspace) || (rows > 0 && (!h || !dy || !dh)))
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": null pointer");
   if (noalloc) {
-    const BwdPlan plan = bwd_plan(h, weight, dy, dh_direct, dh, rows, dim);
+    const BwdPlan plan = bwd_plan(h, weight, dy, dh_direct, dh, rows, dim, x_dtype == FERRITE_BF16 ? 2 : 4,
+                                  dh_dtype == FERRITE_BF16 ? 2 : 4);
     if (plan.bytes > (int64_t)FERRITE_RMSNORM_BWD_SCRATCH_BYTES)
       return fail(FERRITE_ERR_INVALID_ARGUMENT,
                   std::string(name) + ": rows=" + std::to_string(rows) + ", dim=" + std::to_string(dim) + " need " +

@@ -263,3 +263,57 @@ def test_stream_read_and_fill_are_exact(dev, nbytes, blocks):
     o = out.cpu().numpy().view(np.uint32)
     assert np.all(o[:n] == 0x3F803F80) and np.all(o[n:] == 7)
 
+
+
+@pytest.mark.parametrize("rows,dim,dtype", [
+    (5, 1, "f32"), (9, 250, "bf16"), (7, 255, "bf16"),    # a wave per row: pairs and single elements
+    (3, 2046, "bf16"), (5, 1025, "f32"), (6, 1023, "f32"),
+    (6, 4104, "bf16"), (5, 8192, "f32"),                  # a workgroup per row in units of 8
+    (4, 4098, "f32"), (3, 4097, "bf16"), (700, 3001, "f32"),
+    (3, 8200, "bf16"), (2, 16384, "f32"), (3, 8191, "f32"),  # 16 waves per row
+    (3, 16392, "bf16"), (2, 8193, "f32"),                 # wider than any group: the two-sweep kernels
+    (5, 1000, "f32"),                                     # shifted: units of 8 become pairs or single elements
+])
+@pytest.mark.parametrize("shift", [0, 1, 2])
+def test_odd_and_wide_rows(dev, rows, dim, dtype, shift):
+    """Rows outside the fast path, through the C ABI on buffers whose base is `shift` elements past an
+    aligned address: add+norm, norm and the backward with a direct gradient against float64, nothing
+    outside the outputs written. Bars: one rounding of the output type, and f32 sums of dim (rows,
+    for dw) terms."""
+    lib, st = _hip.lib(), torch.cuda.current_stream().cuda_stream
+    dt = torch.float32 if dtype == "f32" else torch.bfloat16
+    code, n = _hip.dtype_code(dt), rows * dim
+    g = torch.Generator(device=dev).manual_seed(rows * dim + shift)
+
+    def place(t):
+        buf = torch.empty(t.numel() + shift, dtype=dt, device=dev)
+        buf[shift:] = t.reshape(-1).to(dt)
+        return buf[shift:]
+
+    x, r, dy, dd = (place(torch.randn(n, device=dev, generator=g)) for _ in range(4))
+    w = place(1 + 0.1 * torch.randn(dim, device=dev, generator=g))
+    outs = [torch.full((n + shift + 8,), float("nan"), dtype=dt, device=dev) for _ in range(4)]
+    h, y, y1, dh = (b[shift:] for b in outs)
+    dw = torch.full((dim + 8,), float("nan"), dtype=dt, device=dev)
+    ws = torch.full((lib.ferrite_hip_rmsnorm_bwd_workspace(rows, dim) // 4,), float("nan"), device=dev)
+    P = [t.data_ptr() for t in (x, r, w, h, y, y1, dy, dd, dh, dw, ws)]
+    _hip.check(lib.ferrite_hip_add_rmsnorm(P[0], P[1], P[2], P[3], P[4], rows, dim, code, code, 1e-6, st), "add")
+    _hip.check(lib.ferrite_hip_rmsnorm(P[0], P[2], P[5], rows, dim, code, code, 1e-6, st), "norm")
+    _hip.check(lib.ferrite_hip_rmsnorm_bwd(P[0], P[2], P[6], P[7], P[8], P[9], P[10], rows, dim, code, code, code, 1e-6,
+                                           st), "bwd")
+    torch.cuda.synchronize()
+    X, R, W, DY, DD = (t.double() for t in (x.view(rows, dim), r.view(rows, dim), w, dy.view(rows, dim), dd.view(rows, dim)))
+
+    def norm(a):
+        return a * torch.rsqrt(a.square().mean(1, keepdim=True) + 1e-6) * W
+
+    inv = torch.rsqrt(X.square().mean(1, keepdim=True) + 1e-6)
+    dxh, xh = DY * W, X * inv
+    dh64 = inv * (dxh - xh * (dxh * xh).mean(1, keepdim=True)) + DD
+    eps = 2.0**-8 if dtype == "bf16" else 2.0**-20
+    for got, ref in ((h, X + R), (y, norm(X + R)), (y1, norm(X)), (dh, dh64)):
+        assert ((got[:n].double().view(rows, dim) - ref).abs() <= eps * ref.abs().clamp(min=1)).all()
+        assert torch.isnan(got[n:]).all()
+    dw64 = (DY * xh).sum(0)
+    assert ((dw[:dim].double() - dw64).abs() <= eps * (DY * xh).abs().sum(0).clamp(min=1)).all()
+    assert torch.isnan(dw[dim:]).all() and all(torch.isnan(b[:shift]).all() for b in outs)
