@@ -7,6 +7,8 @@ Frobenius < 5e-2, prefix invariance). fwd/bwd at
 bf16 outputs and <= 1e-3 for the logsumexp.
 """
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -585,3 +587,50 @@ def test_packed_qkv_argument_errors(dev):
     assert "head_dim" in _hip.last_error()
     assert lib.ferrite_hip_attn_fwd_qkv(x.data_ptr(), o.data_ptr(), lse.data_ptr(), 1, 60, 2, 64, 0.1, st) == 1
     assert "seq" in _hip.last_error()
+
+
+@pytest.mark.parametrize("b,h,sq,sk,d,causal", [
+    (1, 1, 1, 1, 4, True),          # one row: three of the four waves have no tile
+    (1, 2, 33, 33, 32, True),       # a second tile of one row
+    (2, 1, 129, 129, 36, True),     # d between the padded dims; the fifth tile is one wave's second
+    (1, 3, 70, 300, 64, False),     # ragged on both sides, more keys than queries
+    (1, 1, 300, 70, 128, False),
+    (2, 2, 256, 256, 100, True),
+    (1, 130, 128, 128, 64, False),  # 260 workgroups of 128 rows: the other kernels
+    (1, 128, 512, 512, 64, True),   # forward and dQ on the shared sweeps, dK/dV on the other kernels
+])
+@pytest.mark.parametrize("scale", [0.2, -0.3])
+def test_f32_kernels(dev, b, h, sq, sk, d, causal, scale):
+    """Float32 attention, both kernel families and their edges, against float64: outputs to 2e-6 and
+    gradients to 4e-6 of the tensor's largest value, sums of up to 512 f32 products and terms (twice
+    the largest seen), lse to 1e-5; nothing written past the outputs (guards behind each)."""
+    from ferrite import _hip
+
+    g = torch.Generator(device=dev).manual_seed(b * 1000 + sq + d)
+    q, do = (torch.randn(b, h, sq, d, device=dev, generator=g) for _ in range(2))
+    k, v = (torch.randn(b, h, sk, d, device=dev, generator=g) for _ in range(2))
+    lib, st = _hip.lib(), torch.cuda.current_stream().cuda_stream
+    sizes = [q.numel(), b * h * sq, q.numel(), k.numel(), k.numel()]
+    bufs = [torch.full((n + 8,), float("nan"), device=dev) for n in sizes]
+    o, lse, dq, dk, dv = bufs
+    delta = torch.empty(b, h, sq, device=dev)
+    dims = (b, h, sq, sk, d, _hip.F32, int(causal), scale)
+    _hip.check(lib.ferrite_hip_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), *dims,
+                                        st), "fwd")
+    _hip.check(lib.ferrite_hip_attn_bwd_dq_delta(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
+                                                 lse.data_ptr(), delta.data_ptr(), dq.data_ptr(), *dims, st), "dq")
+    _hip.check(lib.ferrite_hip_attn_bwd_dkv(q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), lse.data_ptr(),
+                                            delta.data_ptr(), dk.data_ptr(), dv.data_ptr(), *dims, st), "dkv")
+    torch.cuda.synchronize()
+    Q, K, V, DO = (t.double() for t in (q, k, v, do))
+    s = Q @ K.transpose(-1, -2) * scale
+    if causal:
+        s.masked_fill_(torch.ones(sq, sk, dtype=torch.bool, device=dev).triu_(1), -math.inf)
+    p = torch.softmax(s, -1)
+    O = p @ V
+    ds = p * (DO @ V.transpose(-1, -2) - (DO * O).sum(-1, keepdim=True)) * scale
+    refs = (O, torch.logsumexp(s, -1), ds @ K, ds.transpose(-1, -2) @ Q, p.transpose(-1, -2) @ DO)
+    for name, buf, n, ref, bar in zip(("o", "lse", "dq", "dk", "dv"), bufs, sizes, refs, (2e-6, 1e-5, 4e-6, 4e-6, 4e-6)):
+        err = (buf[:n].double() - ref.reshape(-1)).abs().max() / ref.abs().max().clamp(min=1)
+        assert err <= bar, (name, float(err))
+        assert torch.isnan(buf[n:]).all(), name
