@@ -52,6 +52,8 @@ def linear(x, w):
     """``x @ w`` for ``x: [..., in]`` and ``w: [in, out]`` rounded to x's dtype, as
     ``matmul(x, w.to(x.dtype))`` computes it (model/gpt.py:95-104). Differentiable; a float
     weight's gradient is not rounded."""
+    if x.ndim < 1 or w.ndim != 2 or x.shape[-1] != w.shape[0]:
+        raise ValueError(f"expected [..., in] @ [in, out], got {tuple(x.shape)} @ {tuple(w.shape)}")
     _hip.require_gpu(x, w)
     return _hip.autograd().linear(x, w)
 
@@ -67,6 +69,8 @@ def mlp_gelu(x, w1, w2):
 
 def mlp_gelu_rounded(x, w1, w2):
     """:func:`mlp_gelu` with float32 or bf16 weights, rounded as :func:`linear` rounds its own."""
+    if x.dtype != torch.bfloat16:
+        raise ValueError(f"mlp_gelu takes bf16 x; got {x.dtype}")
     if w1.ndim != 2 or w2.ndim != 2 or x.shape[-1] != w1.shape[0] or w1.shape[1] != w2.shape[0]:
         raise ValueError(f"expected [..., d] @ [d, f] @ [f, e]; got {tuple(x.shape)}, {tuple(w1.shape)}, {tuple(w2.shape)}")
     _hip.require_gpu(x, w1, w2)

@@ -241,3 +241,15 @@ def test_backward_workspace_query():
     assert rc == 1 and "workspace" in _hip.last_error()
     rc = lib.ferrite_hip_attn_bwd_dq_delta_ex(*p, 1, 8, 8192, 8192, 64, bf, 1, 0.125, None, 1024, None)
     assert rc == 1 and "workspace" in _hip.last_error()
+
+
+def test_linear_and_mlp_refuse_what_does_not_match():
+    """Shapes and types are refused before a kernel would read past an operand (no GPU needed)."""
+    from ferrite.kernels.matmul import linear, mlp_gelu_rounded
+
+    bf16 = torch.bfloat16
+    for x, w in (((4, 64), (32, 8)), ((2, 3, 32), (64, 8)), ((4, 64), (64,)), ((4, 64), (2, 64, 8)), ((), (64, 8))):
+        with pytest.raises(ValueError, match="expected"):
+            linear(torch.zeros(x, dtype=bf16), torch.zeros(w))
+    with pytest.raises(ValueError, match="bf16"):
+        mlp_gelu_rounded(torch.zeros(4, 8), torch.zeros(8, 16), torch.zeros(16, 8))
