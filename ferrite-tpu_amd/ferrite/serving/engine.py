@@ -122,10 +122,7 @@ def decode_step(params, token, pos, k_cache, v_cache, cfg: GPTConfig):
     the cache write and the attention; otherwise torch restates the reference's XLA math."""
     b = token.shape[0]
     kernels = cfg.attention == "pallas"
-    if kernels:
-        h = _embed(params, token, pos, cfg)
-    else:
-        h = (params["tok_emb"][token] + params["pos_emb"][pos.long()]).to(cfg.dtype)  # [B, d]
+    h = _embed(params, token, pos, cfg, kernels)
     scale = 1.0 / math.sqrt(cfg.head_dim)
     pending = None
     for i, layer in enumerate(params["layers"]):
@@ -152,10 +149,23 @@ def decode_step(params, token, pos, k_cache, v_cache, cfg: GPTConfig):
     return _dot_f32(y, params["tok_emb"].to(cfg.dtype).t())
 
 
-def _embed(params, token, pos, cfg: GPTConfig):
-    """The decode step's embeddings [B, d] in cfg.dtype, in one kernel."""
-    _hip.require_gpu(token, pos, params["tok_emb"], params["pos_emb"])
-    return _hip.native().embed(token, pos, params["tok_emb"], params["pos_emb"], cfg.dtype)
+def _embed(params, token, pos, cfg: GPTConfig, kernels: bool):
+    """The decode step's embeddings [B, d] in cfg.dtype; in one kernel where the tables are alike and
+    there is one position per token."""
+    tok, pe = params["tok_emb"], params["pos_emb"]
+    if kernels and _one_kernel_embedding(tok, pe, token, pos, cfg.dtype):
+        _hip.require_gpu(token, pos, tok, pe)
+        return _hip.native().embed(token, pos, tok, pe, cfg.dtype)
+    return (tok[token] + pe[pos.long()]).to(cfg.dtype)
+
+
+def _one_kernel_embedding(tok, pe, token, pos, dtype) -> bool:
+    """The kernel reads both tables in one dtype and width, with 64-bit token and 32-bit position indices."""
+    floats = (torch.float32, torch.bfloat16)
+    return (tok.dtype == pe.dtype and tok.dtype in floats and dtype in floats
+            and tok.ndim == pe.ndim == 2 and tok.shape[1] == pe.shape[1] and tok.numel() > 0 and pe.numel() > 0
+            and token.ndim == 1 and pos.shape == token.shape
+            and token.dtype in (torch.int64, torch.int32) and pos.dtype in (torch.int64, torch.int32))
 
 
 def _few_rows_head(y, emb) -> bool:

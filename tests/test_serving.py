@@ -82,3 +82,20 @@ def test_capture_window_holds_off_the_cycle_collector():
         assert not gc.isenabled()
     finally:
         gc.enable()
+
+
+def test_one_kernel_embedding_takes_only_alike_tables():
+    """The decode step's embedding kernel is kept to what it reads: two tables of one dtype and width,
+    a position for each token. Anything else goes through torch's indexing, which is also the result."""
+    from ferrite.serving.engine import _embed, _one_kernel_embedding
+
+    f32, bf16 = torch.float32, torch.bfloat16
+    tok, pe = torch.randn(9, 16), torch.randn(5, 16)
+    t, p = torch.tensor([1, -1, 3]), torch.tensor([0, 4, 2], dtype=torch.int32)
+    assert _one_kernel_embedding(tok, pe, t, p, bf16) and _one_kernel_embedding(tok.bfloat16(), pe.bfloat16(), t, p, f32)
+    for case in ((tok, pe.bfloat16(), t, p), (tok.bfloat16(), pe, t, p), (tok.half(), pe.half(), t, p),
+                 (tok, pe[:, :1], t, p), (tok, pe, t, p[:1]), (tok, pe, t, p[0])):
+        assert not _one_kernel_embedding(*case, bf16)
+        got = _embed({"tok_emb": case[0], "pos_emb": case[1]}, case[2], case[3], CFG.replace(dtype=bf16), True)
+        assert torch.equal(got, (case[0][case[2]] + case[1][case[3].long()]).to(bf16))
+    assert not _one_kernel_embedding(tok, pe, t, p, torch.float16)
