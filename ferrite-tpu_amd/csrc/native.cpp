@@ -344,7 +344,8 @@ struct MatmulFn : torch::autograd::Function<MatmulFn> {
 // 64 rows of bf16 against a float weight read the weight as it is; otherwise a rounded copy is
 // made. The weight's gradient comes back in the weight's own dtype, unrounded if that is float.
 bool reads_f32_weight(const Tensor& x, const Tensor& w) {
-  return x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kFloat && rows_of(x) <= 64;
+  return x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kFloat && rows_of(x) <= 64 &&
+         w.size(0) <= 0x7fffffff / 128 && w.size(1) <= 0x7fffffff / 64;  // skinny_ok
 }
 Tensor linear_f32w(const Tensor& x0, const Tensor& w0, const Tensor& aux) {
   const Tensor x = x0.contiguous(), w = w0.contiguous();
