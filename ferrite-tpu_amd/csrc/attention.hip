@@ -4143,9 +4143,8 @@ int fwd_pp_launch(const void* q, const void* k, const void* v, void* o, float* l
 //   4x16x1024x128 causal (512): 193 / 212, 243 / 300, 341 / 395
 //   4x16x1024x64 causal (512): 113 / 86, 166 / 133, 208 / 222
 // With two waves per SIMD (the forward and dQ up to head dim 64) a causal grid of any size is theirs.
-// Their descriptors span a head's rows from a tile on, which have to stay under 2^31 bytes.
-bool f32_shared_sweeps(int64_t workgroups, int64_t head_elems, int causal, bool two_waves, int64_t cus) {
-  return head_elems < (int64_t)1 << 29 && (workgroups < (causal ? 2 : 1) * cus || (causal && two_waves));
+bool f32_shared_sweeps(int64_t workgroups, int causal, bool two_waves, int64_t cus) {
+  return workgroups < (causal ? 2 : 1) * cus || (causal && two_waves);
 }
 
 // ws / ws_bytes: the caller's workspace for the split long-context forward
@@ -4158,7 +4157,7 @@ int fwd_launch(const void* q, const void* k, const void* v, void* o, float* lse,
   const int64_t bh = s.b * s.h;
   if (nq * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_fwd: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (f32_shared_sweeps(nq * bh, std::max(s.sq, s.sk) * s.d, causal, D <= 64, cu_count(stream)))
+    if (f32_shared_sweeps(nq * bh, causal, D <= 64, cu_count(stream)))
       return f32_attn_fwd(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                           static_cast<float*>(o), lse, {bh, s.sq, s.sk, s.d, causal}, scale, stream);
   }
@@ -4286,7 +4285,7 @@ int dq_launch(const void* q, const void* k, const void* v, const void* dout, con
   const int64_t bh = s.b * s.h;
   if (nq * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_bwd_dq: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (f32_shared_sweeps(nq * bh, std::max(s.sq, s.sk) * s.d, causal, D <= 64, cu_count(stream)))
+    if (f32_shared_sweeps(nq * bh, causal, D <= 64, cu_count(stream)))
       return f32_attn_dq(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                          static_cast<const float*>(dout), lse, delta, static_cast<float*>(dq),
                          {bh, s.sq, s.sk, s.d, causal}, scale, stream);
@@ -4367,7 +4366,7 @@ int dkv_launch(const void* q, const void* k, const void* v, const void* dout, co
   const int64_t bh = s.b * s.h;
   if (nk * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_bwd_dkv: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (f32_shared_sweeps(nk * bh, std::max(s.sq, s.sk) * s.d, causal, false, cu_count(stream)))
+    if (f32_shared_sweeps(nk * bh, causal, false, cu_count(stream)))
       return f32_attn_dkv(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                           static_cast<const float*>(dout), lse, delta, static_cast<float*>(dk),
                           static_cast<float*>(dv), {bh, s.sq, s.sk, s.d, causal}, scale, stream);
