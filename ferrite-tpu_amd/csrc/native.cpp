@@ -341,8 +341,16 @@ struct MatmulFn : torch::autograd::Function<MatmulFn> {
 };
 
 // x @ w with w rounded to x's dtype (model/gpt.py:95-104), for x [..., in] and w [in, out]. Up to
-// 64 rows of bf16 against a float weight read the weight as it is; otherwise a rounded copy is
-// made. The weight's gradient comes back in the weight's own dtype, unrounded if that is float.
+// 64 rows of bf16 against a float weight read the weight as it is, unless a backward is recorded:
+// that one has to find the forward's weight also after an update in place, so it keeps a rounded
+// copy, as larger products do. The weight's gradient comes back in the weight's own dtype,
+// unrounded if that is float.
+bool records(std::initializer_list<const Tensor*> inputs) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : inputs)
+    if (t->requires_grad()) return true;
+  return false;
+}
 bool reads_f32_weight(const Tensor& x, const Tensor& w) {
   return x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kFloat && rows_of(x) <= 64 &&
          w.size(0) <= 0x7fffffff / 128 && w.size(1) <= 0x7fffffff / 64;  // skinny_ok
@@ -359,8 +367,8 @@ Tensor linear_f32w(const Tensor& x0, const Tensor& w0, const Tensor& aux) {
   return out;
 }
 struct LinearFn : torch::autograd::Function<LinearFn> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
-    const bool keep = reads_f32_weight(x, w);
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, bool recorded) {
+    const bool keep = !recorded && reads_f32_weight(x, w);
     const Tensor wq = keep ? w : w.to(x.scalar_type());
     ctx->save_for_backward({x, wq});
     ctx->saved_data["w"] = w.scalar_type();
@@ -373,7 +381,7 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
     const Tensor wq = s[1].to(x.scalar_type()), g = gs[0].to(x.scalar_type());
     const int64_t m = rows_of(x), k = wq.size(0), n = wq.size(1);
     return {mm(g, wq, m, k, n, false, true, x.scalar_type(), x.sizes()),
-            mm(x, g, k, n, m, true, false, ctx->saved_data["w"].toScalarType(), {k, n})};
+            mm(x, g, k, n, m, true, false, ctx->saved_data["w"].toScalarType(), {k, n}), Tensor()};
   }
 };
 
@@ -382,9 +390,9 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
 // Backward: the product g @ w2^T is scaled by gelu'(u) as it is stored, so neither direction runs
 // an elementwise GELU pass.
 struct MlpFn : torch::autograd::Function<MlpFn> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const Tensor& w2) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const Tensor& w2, bool recorded) {
     const int64_t t = rows_of(x), d = w1.size(0), f = w1.size(1), e = w2.size(1);
-    const bool keep = reads_f32_weight(x, w1) && w2.scalar_type() == at::kFloat;
+    const bool keep = !recorded && reads_f32_weight(x, w1) && w2.scalar_type() == at::kFloat;
     Tensor q1 = w1, q2 = w2, u = at::empty({t, f}, x.options()), a, out;
     if (keep) {
       a = linear_f32w(x, w1, u);
@@ -410,13 +418,15 @@ struct MlpFn : torch::autograd::Function<MlpFn> {
     Tensor dw2 = mm(a, g, f, e, t, true, false, ctx->saved_data["w2"].toScalarType(), {f, e});
     Tensor dx = mm(du, q1, t, d, f, false, true, dt, x.sizes());
     Tensor dw1 = mm(x, du, d, f, t, true, false, ctx->saved_data["w1"].toScalarType(), {d, f});
-    return {dx, dw1, dw2};
+    return {dx, dw1, dw2, Tensor()};
   }
 };
 
 Tensor matmul(const Tensor& x, const Tensor& y, at::ScalarType out_dtype) { return MatmulFn::apply(x, y, out_dtype); }
-Tensor linear(const Tensor& x, const Tensor& w) { return LinearFn::apply(x, w); }
-Tensor mlp(const Tensor& x, const Tensor& w1, const Tensor& w2) { return MlpFn::apply(x, w1, w2); }
+Tensor linear(const Tensor& x, const Tensor& w) { return LinearFn::apply(x, w, records({&x, &w})); }
+Tensor mlp(const Tensor& x, const Tensor& w1, const Tensor& w2) {
+  return MlpFn::apply(x, w1, w2, records({&x, &w1, &w2}));
+}
 Tensor mm_2d(const Tensor& x, const Tensor& y, int64_t m, int64_t n, int64_t k, bool x_t, bool y_t,
              at::ScalarType out_dtype) {
   return mm(x, y, m, n, k, x_t, y_t, out_dtype, {m, n});

@@ -51,6 +51,30 @@ def test_mlp_rounds_its_weights(dev, rows):
     assert outs[0][2].dtype == outs[0][3].dtype == torch.float32
 
 
+@pytest.mark.parametrize("rows", [1, 64])
+def test_few_rows_keep_the_forward_weights(dev, rows):
+    """A float weight read in place (no backward recorded) gives the recorded call's output, whose
+    backward uses the weights of the forward also after they were updated in place."""
+    x = _rand(dev, rows, 128, seed=20).requires_grad_()
+    w1 = _rand(dev, 128, 256, seed=21, dtype=torch.float32, scale=0.1).requires_grad_()
+    w2 = _rand(dev, 256, 72, seed=22, dtype=torch.float32, scale=0.1).requires_grad_()
+    g1, g2 = _rand(dev, rows, 256, seed=23), _rand(dev, rows, 72, seed=24)
+    for call, ws, g in ((linear, (w1,), g1), (mlp_gelu_rounded, (w1, w2), g2)):
+        want = torch.autograd.grad(call(x, *ws), (x, *ws), g)
+        y = call(x, *ws)
+        with torch.no_grad():
+            # the same f32 sums up to their order, rounded to bf16 (the MLP: twice)
+            assert (call(x, *ws).float() - y.float()).abs().max() <= 2.0**-7 * y.float().abs().max()
+            keep = [w.clone() for w in ws]
+            for w in ws:
+                w.mul_(2)
+        got = torch.autograd.grad(y, (x, *ws), g)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        with torch.no_grad():
+            for w, k in zip(ws, keep):
+                w.copy_(k)
+
+
 def test_hooks_streams_and_views(dev):
     """Saved-tensor hooks see what is saved, a backward runs on its forward's stream, and
     non-contiguous inputs and gradients give what dense ones do."""
