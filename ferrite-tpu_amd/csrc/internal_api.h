@@ -47,12 +47,24 @@ int ferrite_internal_decode_attention(const void* q, const void* k_new, const vo
 
 /*
  * out[r] = tok_emb[tokens[r]] + pos_emb[pos[r]] for one token per row (model/gpt.py:124-127 at the
- * positions of a decode step), summed and rounded in emb_dtype, then converted to out_dtype.
+ * positions of a decode step; without pos, row r is at position r % period, period <= seq),
+ * summed and rounded in emb_dtype, then converted to out_dtype.
  * tok_emb [vocab, dim], pos_emb [seq, dim]. A negative index counts from the table's end; one
  * outside the table traps, as the gather of a tensor library does.
  */
 int ferrite_internal_embed(const int64_t* tokens, const int32_t* pos, const void* tok_emb, const void* pos_emb, void* out,
-                           int64_t rows, int64_t dim, int64_t vocab, int64_t seq, int emb_dtype, int out_dtype,
-                           void* stream);
+                           int64_t rows, int64_t dim, int64_t vocab, int64_t seq, int64_t period, int emb_dtype,
+                           int out_dtype, void* stream);
+
+/*
+ * Its gradients without pos, summed in f32 in a fixed order: dtok[vocab, dim], the rows of
+ * dh[rows, dim] summed by token, and dpos[seq, dim], by position (zero from period on). Up to 1024
+ * tokens in the vocabulary and whole sequences. The workspace, 16-byte aligned as dtok is, has
+ * ferrite_internal_embed_bwd_workspace(...) bytes (-1: sizes out of range).
+ */
+int64_t ferrite_internal_embed_bwd_workspace(int64_t rows, int64_t period, int64_t dim, int64_t vocab, int64_t seq);
+int ferrite_internal_embed_bwd(const int64_t* tokens, const void* dh, void* dtok, void* dpos, int64_t rows,
+                               int64_t period, int64_t dim, int64_t vocab, int64_t seq, int dh_dtype, int emb_dtype,
+                               void* workspace, int64_t workspace_bytes, void* stream);
 
 }  // extern "C"

@@ -453,10 +453,45 @@ Tensor embed(const Tensor& tokens0, const Tensor& pos0, const Tensor& tok0, cons
   const Tensor tok = tok0.contiguous(), pe = pe0.contiguous();
   Tensor out = at::empty({tokens.numel(), tok.size(1)}, tok.options().dtype(dtype));
   check(ferrite_internal_embed((const int64_t*)ptr(tokens), (const int32_t*)ptr(pos), ptr(tok), ptr(pe), ptr(out),
-                               tokens.numel(), tok.size(1), tok.size(0), pe.size(0), code(tok), code(dtype),
+                               tokens.numel(), tok.size(1), tok.size(0), pe.size(0), 0, code(tok), code(dtype),
                                stream_of(tok)),
         "ferrite_embed");
   return out;
+}
+
+// The embedding of tokens [B, S] (model/gpt.py:124-127) in `dtype`, with the tables' gradients.
+struct EmbedFn : torch::autograd::Function<EmbedFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& tokens0, const Tensor& tok0, const Tensor& pe0,
+                        at::ScalarType dtype) {
+    const Tensor tokens = tokens0.to(at::kLong).contiguous(), tok = tok0.contiguous(), pe = pe0.contiguous();
+    const int64_t dim = tok.size(1);
+    Tensor out = at::empty({tokens.size(0), tokens.size(1), dim}, tok.options().dtype(dtype));
+    check(ferrite_internal_embed((const int64_t*)ptr(tokens), nullptr, ptr(tok), ptr(pe), ptr(out), tokens.numel(), dim,
+                                 tok.size(0), pe.size(0), tokens.size(1), code(tok), code(dtype), stream_of(tok)),
+          "ferrite_embed");
+    ctx->save_for_backward({tokens});
+    ctx->saved_data["vocab"] = tok.size(0);
+    ctx->saved_data["seq"] = pe.size(0);
+    ctx->saved_data["dtype"] = tok.scalar_type();
+    ctx->saved_data["out"] = dtype;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list gs) {
+    const Tensor tokens = ctx->get_saved_variables()[0];
+    const Tensor g = gs[0].to(ctx->saved_data["out"].toScalarType()).contiguous();
+    const int64_t vocab = ctx->saved_data["vocab"].toInt(), seq = ctx->saved_data["seq"].toInt();
+    const int64_t rows = tokens.numel(), period = tokens.size(1), dim = g.size(2);
+    const auto opt = g.options().dtype(ctx->saved_data["dtype"].toScalarType());
+    Tensor dtok = at::empty({vocab, dim}, opt), dpos = at::empty({seq, dim}, opt);
+    const Tensor ws = bytes_on(ferrite_internal_embed_bwd_workspace(rows, period, dim, vocab, seq), g);
+    check(ferrite_internal_embed_bwd((const int64_t*)ptr(tokens), ptr(g), ptr(dtok), ptr(dpos), rows, period, dim, vocab,
+                                     seq, code(g), code(dtok), ptr(ws), size_of(ws), stream_of(g)),
+          "ferrite_embed_bwd");
+    return {Tensor(), dtok, dpos, Tensor()};
+  }
+};
+Tensor embed_tokens(const Tensor& tokens, const Tensor& tok, const Tensor& pe, at::ScalarType dtype) {
+  return EmbedFn::apply(tokens, tok, pe, dtype);
 }
 
 // q, k_new, v_new [B, H, D] are read as they lie when they share one stride per sequence and their
@@ -538,6 +573,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mm", &mm_2d, nogil());
   m.def("tied_logits", &tied_logits, nogil());
   m.def("embed", &embed, nogil());
+  m.def("embed_tokens", &embed_tokens, nogil());
   m.def("decode_attention", &decode_attention, nogil());
   m.def("cross_entropy", &cross_entropy, nogil());
   m.def("cross_entropy_rows", &cross_entropy_rows, nogil());

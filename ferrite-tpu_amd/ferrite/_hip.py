@@ -136,7 +136,12 @@ INTERNAL: dict[str, tuple] = {
     ),
     "ferrite_internal_embed": (
         _c_int,
-        [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _vp],
+        [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _vp],
+    ),
+    "ferrite_internal_embed_bwd_workspace": (_c_i64, [_c_i64] * 5),
+    "ferrite_internal_embed_bwd": (
+        _c_int,
+        [_vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _vp, _c_i64, _vp],
     ),
 }
 

@@ -28,7 +28,7 @@ from typing import Iterator
 import torch
 import torch.nn.functional as F
 
-from ferrite import platform
+from ferrite import _hip, platform
 from ferrite.kernels.flash_attention import (BlockSizes, flash_attention, flash_attention_qkv,
                                             flash_attention_qkv_supported, flash_attention_reference)
 from ferrite.kernels.heads import merge_heads, split_heads
@@ -288,12 +288,27 @@ class _TiedHeadLoss(torch.autograd.Function):
         return torch.mm(g, emb), torch.mm(g.t(), y2), None
 
 
+def _one_kernel_embedding(tok, pe, tokens, dtype) -> bool:
+    """The kernels take tables of one dtype and width with up to 1024 tokens (beyond those the library's
+    sorted sums have few rows per token) and plain indices; a table row per position."""
+    floats = (torch.float32, torch.bfloat16)
+    return (tok.is_cuda and tok.device == pe.device == tokens.device and tok.dtype == pe.dtype
+            and tok.dtype in floats and dtype in floats and tok.ndim == pe.ndim == 2
+            and tok.shape[1] == pe.shape[1] and 0 < tok.shape[0] <= 1024 and 0 < tok.shape[1] <= 1 << 20
+            and tokens.ndim == 2 and tokens.dtype in (torch.int64, torch.int32)
+            and 0 < tokens.numel() < 1 << 30 and tokens.shape[1] <= pe.shape[0] < 1 << 31)
+
+
 def _trunk(params, tokens, cfg: GPTConfig):
     """tokens [B, S] -> final normed hidden states [B*S, d] in cfg.dtype (gpt.py:124-142)."""
     b, s = tokens.shape
     if s > cfg.seq_len:
         raise ValueError(f"sequence {s} longer than cfg.seq_len={cfg.seq_len}")
-    h = (params["tok_emb"][tokens] + params["pos_emb"][:s]).to(cfg.dtype)  # residual stream
+    tok, pe = params["tok_emb"], params["pos_emb"]
+    if cfg.norm == "pallas" and _one_kernel_embedding(tok, pe, tokens, cfg.dtype):
+        h = _hip.autograd().embed_tokens(tokens, tok, pe, cfg.dtype)  # residual stream
+    else:
+        h = (tok[tokens] + pe[:s]).to(cfg.dtype)
     pending = None  # sub-layer output whose residual add is fused into the next norm
     for layer in params["layers"]:
         if pending is None:
