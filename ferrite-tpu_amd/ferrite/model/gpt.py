@@ -289,8 +289,10 @@ class _TiedHeadLoss(torch.autograd.Function):
 
 
 def _one_kernel_embedding(tok, pe, tokens, dtype) -> bool:
-    """The kernels take tables of one dtype and width with up to 1024 tokens (beyond those the library's
-    sorted sums have few rows per token) and plain indices; a table row per position."""
+    """The kernels take tables of one dtype and width with up to 1024 tokens (what a wave's table in LDS
+    holds) and plain indices; a table row per position. us forward and backward on one MI355X,
+    torch's indexing / the kernels: 16384 x 512 over 256 tokens 182 / 64, over 512 144 / 75, over
+    1000 144 / 114; 1024 x 512 over 1000 139 / 63; 128 x 128 over 256 132 / 64."""
     floats = (torch.float32, torch.bfloat16)
     return (tok.is_cuda and tok.device == pe.device == tokens.device and tok.dtype == pe.dtype
             and tok.dtype in floats and dtype in floats and tok.ndim == pe.ndim == 2
