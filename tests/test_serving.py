@@ -99,3 +99,17 @@ def test_one_kernel_embedding_takes_only_alike_tables():
         got = _embed({"tok_emb": case[0], "pos_emb": case[1]}, case[2], case[3], CFG.replace(dtype=bf16), True)
         assert torch.equal(got, (case[0][case[2]] + case[1][case[3].long()]).to(bf16))
     assert not _one_kernel_embedding(tok, pe, t, p, torch.float16)
+
+
+def test_one_kernel_embedding_leaves_other_devices_to_indexing():
+    """Tokens may lie on the CPU beside tables on a GPU: the decode step's embedding kernel does not take
+    them, torch's indexing does. (The meta device stands in for the second one.)"""
+    from ferrite.serving.engine import _one_kernel_embedding
+
+    tok, pe = torch.randn(9, 16), torch.randn(5, 16)
+    t, p = torch.tensor([1, 3]), torch.tensor([0, 4], dtype=torch.int32)
+    assert _one_kernel_embedding(tok, pe, t, p, torch.bfloat16)
+    for at in range(4):
+        case = [tok, pe, t, p]
+        case[at] = case[at].to("meta")
+        assert not _one_kernel_embedding(*case, torch.bfloat16)

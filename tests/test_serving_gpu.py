@@ -216,3 +216,14 @@ def test_decode_embedding_and_head(dev, edt, d):
     ref = y.double() @ tok.bfloat16().double().t()
     bound = 2.0**-20 * (y.double().abs() @ tok.bfloat16().double().abs().t())
     assert ((_hip.native().tied_logits(y, tok).double() - ref).abs() <= bound).all()
+
+
+def test_decode_step_takes_tokens_from_the_cpu(dev):
+    """decode_step indexes the tables on the GPU with token ids on the CPU, as torch's indexing does."""
+    cfg = CFG.replace(dtype=torch.bfloat16, linear="pallas")
+    params = init_params(2, cfg, device=dev)
+    kc, vc = (torch.randn(cfg.n_layer, 3, cfg.n_head, 64, cfg.head_dim, device=dev).to(cfg.dtype) for _ in range(2))
+    token, pos = torch.tensor([5, 200, 31]), torch.tensor([9, 63, 0], dtype=torch.int32, device=dev)
+    want = decode_step(params, token.to(dev), pos, kc.clone(), vc.clone(), cfg)
+    got = decode_step(params, token, pos, kc.clone(), vc.clone(), cfg)
+    assert torch.equal(got, want)  # the embedding is the same sum, rounded the same
