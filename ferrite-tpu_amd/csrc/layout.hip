@@ -257,7 +257,7 @@ extern "C" int ferrite_internal_embed(const int64_t* tokens, const int32_t* pos,
   if (!valid_dtype(emb_dtype) || !valid_dtype(out_dtype))
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": dtype must be FERRITE_F32 or FERRITE_BF16");
   if (rows < 0 || rows > 0x7fffffff || dim < 1 || vocab < 1 || seq < 1 ||
-      (!pos && (period < 1 || period > seq)))
+      (rows > 0 && !pos && (period < 1 || period > seq)))
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": sizes out of range");
   if (rows == 0) return FERRITE_OK;
   if (!tokens || !tok_emb || !pos_emb || !out)

@@ -440,6 +440,7 @@ Tensor tied_logits(const Tensor& y0, const Tensor& emb0) {
   const Tensor y = y0.contiguous(), emb = emb0.contiguous();
   const int64_t m = y.size(0), k = y.size(1), n = emb.size(0);
   Tensor out = at::empty({m, n}, y.options().dtype(at::kFloat));
+  if (m == 0) return out;
   if (emb.scalar_type() != at::kFloat) return mm(y, emb, m, n, k, false, true, at::kFloat, {m, n});
   const Tensor ws = bytes_on(ferrite_internal_linear_f32w_workspace(ptr(y), (const float*)ptr(emb), m, n, k, 1), y);
   check(ferrite_internal_linear_f32w(ptr(y), (const float*)ptr(emb), ptr(out), nullptr, m, n, k, 1, FERRITE_F32, ptr(ws),

@@ -227,3 +227,14 @@ def test_decode_step_takes_tokens_from_the_cpu(dev):
     want = decode_step(params, token.to(dev), pos, kc.clone(), vc.clone(), cfg)
     got = decode_step(params, token, pos, kc.clone(), vc.clone(), cfg)
     assert torch.equal(got, want)  # the embedding is the same sum, rounded the same
+
+
+@pytest.mark.parametrize("edt", [torch.float32, torch.bfloat16])
+def test_decode_step_of_no_sequences(dev, edt):
+    """An empty batch gives logits [0, V], through the few-rows head too."""
+    cfg = CFG.replace(dtype=torch.bfloat16, linear="pallas")
+    params = init_params(2, cfg, device=dev, param_dtype=edt)
+    kc, vc = (torch.zeros(cfg.n_layer, 0, cfg.n_head, 64, cfg.head_dim, device=dev, dtype=cfg.dtype) for _ in range(2))
+    token, pos = (torch.zeros(0, dtype=dt, device=dev) for dt in (torch.long, torch.int32))
+    logits = decode_step(params, token, pos, kc, vc, cfg)
+    assert logits.shape == (0, cfg.vocab_size) and logits.dtype == torch.float32
