@@ -30,6 +30,8 @@ def cross_entropy_rows(logits: torch.Tensor, targets: torch.Tensor):
 
 def cross_entropy_grad(logits, targets, lse, dloss, scale: float, dtype=torch.float32):
     """d(scale * sum(loss)) / d logits times the 0-d device tensor ``dloss``, in ``dtype``."""
+    if logits.ndim != 2:
+        raise ValueError(f"expected logits [N, V]; got {tuple(logits.shape)}")
     _hip.require_gpu(logits, targets, lse, dloss)
     return _hip.native().cross_entropy_grad(logits, targets, lse, dloss, scale, dtype)
 

@@ -253,3 +253,12 @@ def test_linear_and_mlp_refuse_what_does_not_match():
             linear(torch.zeros(x, dtype=bf16), torch.zeros(w))
     with pytest.raises(ValueError, match="bf16"):
         mlp_gelu_rounded(torch.zeros(4, 8), torch.zeros(8, 16), torch.zeros(16, 8))
+
+
+@pytest.mark.parametrize("shape", [(8,), (2, 3, 8)])
+def test_cross_entropy_grad_takes_two_dims(shape):
+    """Logits that are not [N, V] are refused before dispatch: the kernel would write a part of the gradient."""
+    from ferrite.kernels.cross_entropy import cross_entropy_grad
+
+    with pytest.raises(ValueError, match="logits"):
+        cross_entropy_grad(torch.zeros(shape), torch.zeros(2, dtype=torch.long), torch.zeros(2), torch.ones(()), 1.0)
