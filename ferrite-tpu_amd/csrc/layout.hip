@@ -133,6 +133,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const int64_t* __restrict__ 
 // chain of table updates in a wave: LDS atomics took 59 us for 16384 x 512 bf16 over 256 tokens,
 // reads and writes of two rows at a time 34. Training step of that size, tables' indexing in
 // torch / these kernels: 2894 / 2841 us.
+constexpr int64_t kMostBlocks = 0xffffffff / 256;  // blocks of 256 threads: a launch has under 2^32 threads along x
 constexpr int kEmbedLds = 64 << 10;
 constexpr int64_t kEmbedVocab = 1024;
 constexpr int kEmbedBatch = 64;  // rows whose loads go out together, a token per lane
@@ -202,7 +203,7 @@ struct EmbedBwd {
   int64_t slab;  // floats from one slice's table to the next
 };
 bool embed_bwd_plan(int64_t rows, int64_t period, int64_t dim, int64_t vocab, int64_t seq, EmbedBwd& p) {
-  if (rows < 1 || rows > 0x3fffffff || period < 1 || rows % period || seq < period || seq > 0x7fffffff || dim < 1 ||
+  if (rows < 1 || rows > 0x3fffffff || period < 1 || rows % period || seq < period || seq > kMostBlocks || dim < 1 ||
       dim > 64 * 65535 || vocab < 1 || vocab > kEmbedVocab)
     return false;
   p.cols = vocab <= 256 ? 64 : vocab <= 512 ? 32 : 16;
@@ -256,7 +257,7 @@ extern "C" int ferrite_internal_embed(const int64_t* tokens, const int32_t* pos,
   const char* name = "ferrite_internal_embed";
   if (!valid_dtype(emb_dtype) || !valid_dtype(out_dtype))
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": dtype must be FERRITE_F32 or FERRITE_BF16");
-  if (rows < 0 || rows > 0x7fffffff || dim < 1 || vocab < 1 || seq < 1 ||
+  if (rows < 0 || rows > kMostBlocks || dim < 1 || vocab < 1 || seq < 1 ||
       (rows > 0 && !pos && (period < 1 || period > seq)))
     return fail(FERRITE_ERR_INVALID_ARGUMENT, std::string(name) + ": sizes out of range");
   if (rows == 0) return FERRITE_OK;

@@ -290,7 +290,8 @@ class _TiedHeadLoss(torch.autograd.Function):
 
 def _one_kernel_embedding(tok, pe, tokens, dtype) -> bool:
     """The kernels take tables of one dtype and width with up to 1024 tokens (what a wave's table in LDS
-    holds) and plain indices; a table row per position. us forward and backward on one MI355X,
+    holds) and plain indices; a table row per position; a block per token and position, in one launch
+    under 2^32 threads. us forward and backward on one MI355X,
     torch's indexing / the kernels: 16384 x 512 over 256 tokens 182 / 64, over 512 144 / 75, over
     1000 144 / 114; 1024 x 512 over 1000 139 / 63; 128 x 128 over 256 132 / 64."""
     floats = (torch.float32, torch.bfloat16)
@@ -298,7 +299,7 @@ def _one_kernel_embedding(tok, pe, tokens, dtype) -> bool:
             and tok.dtype in floats and dtype in floats and tok.ndim == pe.ndim == 2
             and tok.shape[1] == pe.shape[1] and 0 < tok.shape[0] <= 1024 and 0 < tok.shape[1] <= 1 << 20
             and tokens.ndim == 2 and tokens.dtype in (torch.int64, torch.int32)
-            and 0 < tokens.numel() < 1 << 30 and tokens.shape[1] <= pe.shape[0] < 1 << 31)
+            and 0 < tokens.numel() < 1 << 24 and tokens.shape[1] <= pe.shape[0] < 1 << 24)
 
 
 def _trunk(params, tokens, cfg: GPTConfig):

@@ -161,11 +161,13 @@ def _embed(params, token, pos, cfg: GPTConfig, kernels: bool):
 
 def _one_kernel_embedding(tok, pe, token, pos, dtype) -> bool:
     """The kernel reads both tables in one dtype and width, with 64-bit token and 32-bit position indices,
-    all on one device (torch's indexing takes tokens from the CPU too)."""
+    all on one device (torch's indexing takes tokens from the CPU too), a block per token in one launch of
+    under 2^32 threads."""
     floats = (torch.float32, torch.bfloat16)
-    return (tok.device == pe.device == token.device == pos.device and tok.dtype == pe.dtype and tok.dtype in floats and dtype in floats
+    return (tok.device == pe.device == token.device == pos.device
+            and tok.dtype == pe.dtype and tok.dtype in floats and dtype in floats
             and tok.ndim == pe.ndim == 2 and tok.shape[1] == pe.shape[1] and tok.numel() > 0 and pe.numel() > 0
-            and token.ndim == 1 and pos.shape == token.shape
+            and token.ndim == 1 and token.shape[0] < 1 << 24 and pos.shape == token.shape
             and token.dtype in (torch.int64, torch.int32) and pos.dtype in (torch.int64, torch.int32))
 
 

@@ -58,3 +58,29 @@ def test_internal_entry_points_match_their_header():
     text = open(os.path.join(ROOT, "ferrite-tpu_amd", "csrc", "internal_api.h")).read()
     declared = set(re.findall(r"^(?:int|int64_t) (ferrite_internal_\w+)\(", text, re.M))
     assert declared == set(_hip.INTERNAL) and not declared & set(_hip.SIGNATURES)
+
+
+def test_embedding_rules_stay_within_a_launch():
+    """A block of 256 threads per token and position, and under 2^32 threads along a grid's x: the rules
+    leave more to torch's indexing, and the entry points refuse it before a launch."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from ferrite import _hip
+    from ferrite.model import gpt
+    from ferrite.serving import engine
+
+    def tensor(*shape, dtype=torch.float32):
+        return SimpleNamespace(shape=shape, ndim=len(shape), dtype=dtype, device="cuda:0", is_cuda=True,
+                               numel=lambda: int(torch.Size(shape).numel()))
+
+    i64, bf16, most = torch.int64, torch.bfloat16, (1 << 24) - 1
+    for n, takes in ((most, True), (most + 1, False)):
+        assert gpt._one_kernel_embedding(tensor(256, 8), tensor(4, 8), tensor(n, 1, dtype=i64), bf16) == takes
+        assert gpt._one_kernel_embedding(tensor(256, 8), tensor(n, 8), tensor(3, 4, dtype=i64), bf16) == takes
+        assert engine._one_kernel_embedding(tensor(256, 8), tensor(4, 8), tensor(n, dtype=i64), tensor(n, dtype=i64),
+                                            bf16) == takes
+        assert _hip.lib().ferrite_internal_embed(None, None, None, None, None, n, 8, 256, 4, 4, 0, 0, None) == 1
+        assert ("null" if takes else "sizes") in _hip.last_error()
+        assert (_hip.lib().ferrite_internal_embed_bwd_workspace(12, 4, 8, 256, n) > 0) == takes
