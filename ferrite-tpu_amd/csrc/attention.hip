@@ -4132,21 +4132,6 @@ int fwd_pp_launch(const void* q, const void* k, const void* v, void* o, float* l
   return check_launch("ferrite_flash_attention_fwd");
 }
 
-// Whether an f32 pass takes the kernels whose waves share a sweep (attn_f32.hip) rather than those
-// with 128 rows a workgroup, given the latter's grid. Theirs is the better rate once they fill the
-// chip evenly, their waves sharing tiles through LDS: from a workgroup per CU on without a mask,
-// from two with one (whose sweeps differ in length). us on one MI355X, 128 rows / shared sweeps:
-//   2x8x1024x64 causal (128 workgroups): forward 82 / 34, dQ 119 / 50, dK/dV 155 / 62
-//   1x8x4096x64 causal (256): 308 / 158, 459 / 235, 606 / 356
-//   2x8x1024x128 (128): 137 / 92, 211 / 126, 293 / 164
-//   8x16x256x64 (256): 25 / 29, 35 / 44, 47 / 62
-//   4x16x1024x128 causal (512): 193 / 212, 243 / 300, 341 / 395
-//   4x16x1024x64 causal (512): 113 / 86, 166 / 133, 208 / 222
-// With two waves per SIMD (the forward and dQ up to head dim 64) a causal grid of any size is theirs.
-bool f32_shared_sweeps(int64_t workgroups, int causal, bool two_waves, int64_t cus) {
-  return workgroups < (causal ? 2 : 1) * cus || (causal && two_waves);
-}
-
 // ws / ws_bytes: the caller's workspace for the split long-context forward
 // (fwd_split_bytes), or nullptr.
 template <typename T, int D, bool AL>
@@ -4157,7 +4142,7 @@ int fwd_launch(const void* q, const void* k, const void* v, void* o, float* lse,
   const int64_t bh = s.b * s.h;
   if (nq * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_fwd: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (f32_shared_sweeps(nq * bh, causal, D <= 64, cu_count(stream)))
+    if (sched::f32_shared_sweeps(nq * bh, causal, D <= 64, cu_count(stream)))
       return f32_attn_fwd(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                           static_cast<float*>(o), lse, {bh, s.sq, s.sk, s.d, causal}, scale, stream);
   }
@@ -4285,7 +4270,7 @@ int dq_launch(const void* q, const void* k, const void* v, const void* dout, con
   const int64_t bh = s.b * s.h;
   if (nq * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_bwd_dq: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (f32_shared_sweeps(nq * bh, causal, D <= 64, cu_count(stream)))
+    if (sched::f32_shared_sweeps(nq * bh, causal, D <= 64, cu_count(stream)))
       return f32_attn_dq(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                          static_cast<const float*>(dout), lse, delta, static_cast<float*>(dq),
                          {bh, s.sq, s.sk, s.d, causal}, scale, stream);
@@ -4366,7 +4351,7 @@ int dkv_launch(const void* q, const void* k, const void* v, const void* dout, co
   const int64_t bh = s.b * s.h;
   if (nk * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_bwd_dkv: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (f32_shared_sweeps(nk * bh, causal, false, cu_count(stream)))
+    if (sched::f32_shared_sweeps(nk * bh, causal, false, cu_count(stream)))
       return f32_attn_dkv(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                           static_cast<const float*>(dout), lse, delta, static_cast<float*>(dk),
                           static_cast<float*>(dv), {bh, s.sq, s.sk, s.d, causal}, scale, stream);

@@ -142,6 +142,22 @@ FERRITE_SCHED int fwd_split_cut(long long bh, long long S, int cus) { return spl
 // `per_cu` workgroups per CU: when all of them are resident at once.
 FERRITE_SCHED bool resident(long long grid, int per_cu, int cus) { return grid <= (long long)per_cu * cus; }
 
+// Whether an f32 pass takes the kernels whose waves share a sweep (attn_f32.hip) rather than those
+// with 128 rows a workgroup, given the latter's grid. Theirs is the better rate once they fill the
+// chip evenly, their waves sharing tiles through LDS: from a workgroup per CU on without a mask,
+// from two with one (whose sweeps differ in length). us on one MI355X, 128 rows / shared sweeps:
+//   2x8x1024x64 causal (128 workgroups): forward 82 / 34, dQ 119 / 50, dK/dV 155 / 62
+//   1x8x4096x64 causal (256): 308 / 158, 459 / 235, 606 / 356
+//   2x8x1024x128 (128): 137 / 92, 211 / 126, 293 / 164
+//   8x16x256x64 (256): 25 / 29, 35 / 44, 47 / 62
+//   4x16x1024x128 causal (512): 193 / 212, 243 / 300, 341 / 395
+//   4x16x1024x64 causal (512): 113 / 86, 166 / 133, 208 / 222
+// With two waves per SIMD (the forward and dQ up to head dim 64) a causal grid is theirs while their
+// four workgroups of 32 rows for one of 128, of 256 threads each, stay under a launch's 2^32 threads.
+FERRITE_SCHED bool f32_shared_sweeps(long long workgroups, int causal, bool two_waves, long long cus) {
+  return workgroups < (causal ? 2 : 1) * cus || (causal && two_waves && workgroups < 1LL << 22);
+}
+
 // ---- rings -------------------------------------------------------------------
 // Forward (attn_fwd_sw_kernel), SLOTS = 3 (D <= 128) or 2 (D = 256, whose
 // 64-key K and V tiles take 68 KB a slot), tile t in slot t % SLOTS. Stage j

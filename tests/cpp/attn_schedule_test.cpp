@@ -621,12 +621,30 @@ static void check_wide(int bh, int S, int D) {
   }
 }
 
+// The f32 kernels with shared sweeps (f32_shared_sweeps): a workgroup of 256 threads per 32 rows, under 2^32
+// threads along x for every grid the rule gives them.
+static void check_f32_grids() {
+  for (int causal : {0, 1})
+    for (bool two_waves : {false, true})
+      for (long long nq : {1LL, 3LL, 64LL})
+        for (long long bh = 1; nq * bh < 1LL << 24; bh = bh * 3 / 2 + 1)
+          for (long long b : {bh, (1LL << 22) / nq, (1LL << 22) / nq - 1}) {
+            const long long S = 128 * nq;
+            if (f32_shared_sweeps(nq * b, causal, two_waves, kCus) && (S + 31) / 32 * b * 256 >= 1LL << 32)
+              fail("f32: the grid of " + std::to_string(b) + " heads of " + std::to_string(S) + " rows is too large");
+          }
+  if (!f32_shared_sweeps(256, 1, false, kCus) || !f32_shared_sweeps(1 << 20, 1, true, kCus) ||
+      f32_shared_sweeps(256, 0, true, kCus) || f32_shared_sweeps(512, 1, false, kCus))
+    fail("f32: the sweeps are shared on the wrong grids");
+}
+
 int main() {
   std::vector<int> lengths;
   for (int s = 64; s <= 4096; s += 64) lengths.push_back(s);
   lengths.push_back(8192);
   const int bhs[] = {1, 3, 8, 64};
   int launches = 0;
+  check_f32_grids();
   for (int bh : bhs)
     for (int S : lengths) {
       // The forward's launch choices (fwd_launch): D = 128 one 8-wave workgroup per CU; D <= 64 the
