@@ -43,6 +43,7 @@ constexpr int kUnroll = 4;        // row steps whose loads are issued together
 // 2x8x2048x64 took 14.7 us, 7.8 in two passes).
 constexpr int kChunkMin = 128;
 constexpr int64_t kGridTarget = 512;
+constexpr int64_t kNoWorkspaceRows = 256;  // caches of up to here need no workspace: without one they are not cut
 
 template <typename T>
 struct Vec16 {
@@ -313,7 +314,8 @@ int decode_launch(const void* q, const void* kn, const void* vn, void* kc, void*
   constexpr int kStep = kStepRows<T, D>;
   int64_t nch = chunks_for(B, H, L);
   const bool one_group = nch > 1 && L <= 16 * 2 * kStep;
-  if (one_group) nch = 1;
+  const bool fits = ws && ws_bytes >= B * H * nch * (D + 2) * (int64_t)sizeof(float);
+  if (one_group || (!fits && L <= kNoWorkspaceRows)) nch = 1;
   const int wave_rows = (int)(cdiv(cdiv(L, nch * (one_group ? 16 : 4)), (int64_t)kStep) * kStep);
   const float c = scale * kLog2e;
   const dim3 grid((unsigned)nch, (unsigned)H, (unsigned)B);
@@ -330,7 +332,7 @@ int decode_launch(const void* q, const void* kn, const void* vn, void* kc, void*
     hipLaunchKernelGGL((decode_attn_kernel<T, D, true, 4>), grid, dim3(256), 0, st, tq, tk, tv, ck, cv, pos, to,
                        nullptr, (int)L, c, new_stride, wave_rows);
   } else {
-    if (!ws || ws_bytes < B * H * nch * (D + 2) * (int64_t)sizeof(float))
+    if (!fits)
       return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_decode_attention: workspace too small");
     hipLaunchKernelGGL((decode_attn_kernel<T, D, false, 4>), grid, dim3(256), 0, st, tq, tk, tv, ck, cv, pos, to,
                        static_cast<float*>(ws), (int)L, c, new_stride, wave_rows);

@@ -238,3 +238,27 @@ def test_decode_step_of_no_sequences(dev, edt):
     token, pos = (torch.zeros(0, dtype=dt, device=dev) for dt in (torch.long, torch.int32))
     logits = decode_step(params, token, pos, kc, vc, cfg)
     assert logits.shape == (0, cfg.vocab_size) and logits.dtype == torch.float32
+
+
+@pytest.mark.parametrize("L", [129, 256])
+@pytest.mark.parametrize("d,dtype", [(256, torch.float32), (256, torch.bfloat16), (64, torch.float32)])
+def test_decode_attention_of_a_short_cache_needs_no_workspace(dev, L, d, dtype):
+    """The entry point takes caches of up to 256 rows without a workspace, and a longer one that it cuts
+    only with one."""
+    from ferrite import _hip
+
+    def call(length, q, kn, vn, kc, vc, pos):
+        out = torch.full_like(q, float("nan"))
+        return out, _hip.lib().ferrite_hip_decode_attention(
+            *(t.data_ptr() for t in (q, kn, vn, kc, vc, pos, out)), 2, 3, length, d, _hip.dtype_code(dtype), d**-0.5,
+            None, 0, _hip.stream_of(q))
+
+    q, kn, vn, kc, vc = _case(dev, 2, 3, L, d, dtype, L + d)
+    pos = torch.tensor([L - 1, 5], dtype=torch.int32, device=dev)
+    ref = decode_attention_reference(q, kn, vn, kc.clone(), vc.clone(), pos)
+    out, rc = call(L, q, kn, vn, kc, vc, pos)
+    _hip.check(rc, "decode")
+    bar = 2.0**-7 if dtype == torch.bfloat16 else 1e-5  # two f32 sums, and one rounding to bf16 each
+    assert ((out.float() - ref.float()).abs() <= bar * ref.float().abs() + 1e-5).all()
+    q, kn, vn, kc, vc = _case(dev, 2, 3, 2000, d, dtype, 1)
+    assert call(2000, q, kn, vn, kc, vc, pos)[1] == 1 and "workspace" in _hip.last_error()
