@@ -113,6 +113,52 @@ def test_gelu_grad_epilogue(dev, m, n, k):
     assert np.all(np.abs(got - exact) <= bf16_ulp(exact) + 1e-6 * np.abs(exact) + 4e-7 * np.abs(p64) * (1 + u64**2))
 
 
+FEW_ROWS = [  # csrc/skinny.hip: (m, n, k, workspace)
+    (1, 8, 64, True),
+    (8, 264, 128, True),
+    (33, 72, 64, True),     # one row in the second block of 32
+    (64, 3072, 768, True),
+    (8, 512, 4096, True),   # K split: the epilogue in the slices' sum
+    (64, 512, 2048, True),  # K split with two row blocks
+    (8, 512, 4096, False),  # the same product unsplit
+    (7, 27, 4100, True),    # m n not a multiple of 4: unsplit
+    (5, 33, 77, True),      # rows not aligned: element loads
+    (40, 33, 77, True),
+]
+
+
+# A transposed operand takes k in whole 64s and n in whole 8s.
+@pytest.mark.parametrize("m,n,k,workspace,y_t", [(*c, t) for c in FEW_ROWS for t in (False, True)
+                                                if not t or (c[2] % 64 == 0 and c[1] % 8 == 0)])
+def test_few_rows_epilogues(dev, m, n, k, workspace, y_t):
+    """Both epilogues of products of up to 64 rows against f64: the pre-activation is the product to f32
+    sums and one rounding, gelu of it as for the other kernels, and the gradient pass multiplies the
+    rounded product by gelu' of an aux that it leaves alone."""
+    a, b = normal(160 + m, (m, k), "bf16"), normal(161 + n, (k, n), "bf16", scale=k**-0.5)
+    xs, ys = to_dev(a, "bf16", dev), to_dev(b.T.copy() if y_t else b, "bf16", dev)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    exact = a @ b
+    sums = (k + 16) * 2.0**-24 * (np.abs(a) @ np.abs(b))  # f32 sums of k products in any order
+
+    u = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=dev)
+    out = _call(xs, ys, m, n, k, False, y_t, _hip.GELU, u, workspace)
+    torch.cuda.synchronize()
+    un, got = to_np(u).astype(np.float64), to_np(out).astype(np.float64)
+    assert np.all(np.abs(un - exact) <= sums + bf16_ulp(np.abs(exact) + sums))
+    want = _gelu64(un)
+    assert np.all(np.abs(got - want) <= _fwd_bar(want, un))
+
+    un = normal(162, (m, n), "bf16", scale=2.0)
+    aux = to_dev(un, "bf16", dev)
+    out = _call(xs, ys, m, n, k, False, y_t, _hip.GELU_GRAD, aux, workspace)
+    torch.cuda.synchronize()
+    assert np.array_equal(to_np(aux), un)
+    un, got = un.astype(np.float64), to_np(out).astype(np.float64)
+    d = _gelu_grad64(un)
+    slack = np.abs(d) * (sums + bf16_ulp(np.abs(exact) + sums)) + 4e-7 * np.abs(exact) * (1 + un**2)
+    assert np.all(np.abs(got - exact * d) <= slack + bf16_ulp(np.abs(exact * d) + slack))
+
+
 def test_split_and_unsplit_agree(dev):
     """Without a workspace the few-tile shape does not split; both results hold the same bar."""
     m, n, k = 768, 768, 4096
@@ -146,7 +192,7 @@ def test_argument_errors(dev):
     assert "mode" in _hip.last_error()
 
 
-@pytest.mark.parametrize("t,d,f", [(2048, 768, 3072), (384, 256, 1024), (200, 64, 136)])
+@pytest.mark.parametrize("t,d,f", [(2048, 768, 3072), (384, 256, 1024), (200, 64, 136), (8, 256, 1024), (64, 768, 3072)])
 def test_mlp_matches_unfused(dev, t, d, f):
     """mlp_gelu against matmul -> torch's tanh GELU -> matmul on the same bf16 values: output and
     the three gradients within the bf16 bar (2 ulp of the larger magnitude, relative Frobenius 1e-2)."""
