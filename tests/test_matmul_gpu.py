@@ -440,3 +440,31 @@ def test_few_rows(dev, m, n, k, y_t):
         assert torch.equal(o.view(-1), buf[: m * n]) and torch.equal(u, o)
         gelu = torch.nn.functional.gelu(u.double(), approximate="tanh")
         assert ((o2.double() - gelu).abs() <= 2.0**-8 * gelu.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 203, 77), (300, 1003, 130), (129, 520, 63)])
+def test_unaligned_products_without_a_workspace(dev, m, n, k):
+    """ferrite_hip_matmul has no workspace to pack unaligned rows into: more than 64 of them keep the
+    kernel that loads by elements."""
+    a, b, exact, bound = _exact_case(m, n, k)
+    xs, ys = to_dev(a, "bf16", dev), to_dev(b, "bf16", dev)
+    for dt in (torch.float32, torch.bfloat16):
+        buf = torch.full((m * n + 8,), float("nan"), dtype=dt, device=dev)
+        _hip.check(_hip.lib().ferrite_hip_matmul(xs.data_ptr(), ys.data_ptr(), buf.data_ptr(), m, n, k, _hip.BF16,
+                                                 _hip.dtype_code(dt), _hip.stream_of(xs)), "matmul")
+        got = to_np(buf[: m * n]).astype(np.float64).reshape(m, n)
+        assert np.all(np.abs(got - exact) <= bound + (bf16_ulp(exact) if dt == torch.bfloat16 else 0.0))
+        assert torch.isnan(buf[m * n :]).all()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_rows_past_the_buffer_range(dev, dt):
+    """Aligned operands whose 64 rows of n columns pass a buffer's 2^31 bytes: the 64-bit kernel takes them,
+    exactly for whole numbers this small."""
+    m, n, k = 65, 16_800_000, 8
+    g = torch.Generator(device=dev).manual_seed(7)
+    x, y = (torch.randint(-2, 3, s, device=dev, generator=g, dtype=torch.int8).to(torch.bfloat16) for s in ((m, k), (k, n)))
+    out = matmul(x, y, out_dtype=dt)
+    xf = x.float()
+    for c in range(0, n, 1 << 20):
+        assert torch.equal(out[:, c : c + (1 << 20)].float(), xf @ y[:, c : c + (1 << 20)].float())
