@@ -58,7 +58,7 @@ def test_fused_residual_forward(dev):
 
 @pytest.mark.parametrize("rows,dim", [(1, 1024), (3, 1024), (37, 100), (8, 8192), (5, 4096), (64, 2048), (16, 8)])
 def test_shapes_and_paths(dev, rows, dim):
-    """Vector path (dim % 8 == 0, dim <= 4096), generic path (other dims), odd row counts."""
+    """One wave per row in 16-byte vectors (dim % 8 == 0, dim <= 4096), thread groups (other dims), odd row counts."""
     x, r = normal(7, (rows, dim), "bf16"), normal(8, (rows, dim), "bf16")
     w = normal(9, (dim,), "bf16", loc=1.0, scale=0.1)
     h, y = rmsnorm(to_dev(x, "bf16", dev), to_dev(w, "bf16", dev), residual=to_dev(r, "bf16", dev))
@@ -153,9 +153,11 @@ def _bwd_abi(h, w, dy, dd, dh_dtype, dim_slice=None):
     (4096, 1024, "bf16", True),
     (333, 4096, "f32", True),     # VPL 8, ragged row count
     (77, 64, "f32", False),       # VPL 1 with idle lanes
-    (50, 100, "f32", True),       # dim % 8 != 0: general row pass + column pass
-    (19, 5000, "bf16", False),    # dim above the register path: general
+    (50, 100, "f32", True),       # dim % 8 != 0: a wave per row in pairs
+    (19, 5000, "bf16", False),    # wider than the one-pass kernel: a workgroup per row
     (3, 768, "bf16", True),       # fewer rows than waves
+    (4100, 1027, "bf16", True),   # many odd bf16 rows: general row pass + column pass
+    (600, 16392, "f32", False),   # wider than any group: general, more rows than partial rows
 ])
 def test_bwd_kernel_matches_oracle(dev, rows, dim, dtype, direct):
     """dh and dweight of ferrite_hip_rmsnorm_bwd against the f64 analytic backward

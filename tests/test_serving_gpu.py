@@ -3,7 +3,7 @@
 
 Pins for the kernel: the reference's own math (engine.py:89-104: write the new
 rows, f32 scores over keys <= pos masked with -1e30, softmax, P.V), restated in
-torch on the same inputs, at positions on and across the 256-key chunk edges;
+torch on the same inputs, at positions on and across the edges of waves' and workgroups' rows;
 the caches hold the new rows at pos and nothing else changed; out-of-range
 positions write nothing and give NaN; reruns are bitwise equal. For the engine:
 greedy tokens equal re-running the full model per step (the reference's own
@@ -34,7 +34,7 @@ def _case(dev, b, h, L, d, dtype, seed):
     (2, 3, 1000, 64, torch.bfloat16, [0, 999]),
     (2, 3, 1000, 64, torch.bfloat16, [255, 256]),
     (3, 2, 600, 128, torch.bfloat16, [511, 1, 300]),
-    (1, 2, 256, 128, torch.float32, [100]),       # one chunk: direct output
+    (1, 2, 256, 128, torch.float32, [100]),       # one workgroup of 16 waves: direct output
     (2, 1, 300, 256, torch.bfloat16, [257, 299]),
     (4, 12, 2048, 64, torch.float32, [2047, 1024, 3, 1500]),
     # 128 heads: 1024-key chunks (the grid within 512 workgroups)

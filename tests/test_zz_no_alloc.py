@@ -47,7 +47,8 @@ def _run(dev, h, dy, w, dd, rows, dim, xd, wd, od, noalloc):
     ((8192, 768), (1000, 512), "bf16", "f32", "bf16", True),   # the GPT step's norms, fast path
     ((8192, 4096), (64, 1024), "bf16", "bf16", "bf16", False),  # the largest fast-path dim: 512 x 4096 floats = 8 MiB
     ((3000, 1000), (77, 136), "f32", "f32", "f32", False),     # f32, fast path
-    ((700, 100), (33, 60), "bf16", "f32", "f32", True),        # dim % 8 != 0: general row + column passes
+    ((700, 100), (33, 60), "bf16", "f32", "f32", True),        # dim % 8 != 0: thread groups
+    ((4100, 1027), (33, 60), "bf16", "f32", "f32", True),      # many odd bf16 rows: general row + column passes
 ])
 def test_noalloc_matches_workspace_entry(dev, first, second, xd, wd, od, direct):
     for i, (rows, dim) in enumerate((first, second)):
@@ -60,7 +61,7 @@ def test_noalloc_matches_workspace_entry(dev, first, second, xd, wd, od, direct)
 
 
 def test_noalloc_refuses_shapes_beyond_its_scratch(dev):
-    """dim 8192 is past the one-pass kernel's 4096, so 4112 rows take the general path: 512 partial
+    """dim 8192 is past the one-pass kernel's 4096, so 4112 rows count as the general path's: 512 partial
     rows of 8192 floats plus one float per row, (512 * 8192 + 4112) * 4 = 16.8 MB > 8 MiB. Refused
     before any launch, outputs untouched."""
     rows, dim = 4112, 8192
@@ -77,7 +78,8 @@ def test_noalloc_refuses_shapes_beyond_its_scratch(dev):
 
 
 def test_noalloc_scratch_edge_on_the_general_path(dev):
-    """The refusal edge of the general path (dim % 8 != 0): nparts = min(rows, 512) partial rows of
+    """The refusal edge of rows that the one-pass kernel does not take (dim % 8 != 0), counted as the
+    general path's whether a group takes them or not: nparts = min(rows, 512) partial rows of
     dim floats plus one float per row. dim 4095 with 512 rows needs (512 * 4095 + 512) * 4 bytes,
     exactly the 8 MiB array: accepted and bitwise equal to the workspace entry. 513 rows need four
     bytes more: refused, outputs untouched."""
