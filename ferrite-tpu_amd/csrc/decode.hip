@@ -36,12 +36,18 @@ constexpr int kUnroll = 4;        // row steps whose loads are issued together
 // bf16 162.4 us, 32x32x2048x128 bf16 160.2 us, 8x16x8192x128 f32 155.3 us,
 // 1x32x8192x128 bf16 20 us.
 //
-// Grids of few workgroups are bound by latency. Chunks down to 128 keys shorten a wave's
-// chain of loads (3x5x900x256 f32 26.7 -> 17.7 us, 1x1x6590x256 bf16 19.0 -> 17.4 us); where
-// one workgroup of 16 waves reaches the whole cache in two batches of loads a wave, it
+// Grids of few workgroups are bound by latency. Chunks of 128 keys shorten a wave's chain of
+// loads, and add a round trip of the second pass, which reads 8 chunks at a time, for every
+// 8 more of them. They pay up to one chunk per 4 bytes of a row: us on one MI355X, chunks of
+// 256 / 128, on the left of that line and past it:
+//   bf16 1x3x4096x64 8.7 / 8.8     1x3x6000x64 9.6 / 10.5     1x3x16384x64 11.8 / 15.9
+//   f32 1x1x8192x64 12.5 / 11.8    1x1x10000x64 12.3 / 13.2   1x1x16384x64 14.1 / 15.5
+//   bf16 1x1x6000x256 19.5 / 15.7  f32 1x1x16384x128 20.8 / 20.2, 1x1x16384x256 34.3 / 27.7
+// Where one workgroup of 16 waves reaches the whole cache in two batches of loads a wave, it
 // does, and there is no second pass (8x4x512x128 12.1 -> 9.3 us; with four batches a wave
 // 2x8x2048x64 took 14.7 us, 7.8 in two passes).
 constexpr int kChunkMin = 128;
+constexpr int kRowBytesPerChunk = 4;
 constexpr int64_t kGridTarget = 512;
 constexpr int64_t kNoWorkspaceRows = 256;  // caches of up to here need no workspace: without one they are not cut
 
@@ -250,8 +256,9 @@ __global__ __launch_bounds__(64 * WAVES) void decode_attn_kernel(const T* __rest
 }
 
 // One block per head: merge the chunks that hold keys (0..pos) and normalise.
-// Loads go out eight chunks at a time, so a thread waits on a few batches of
-// independent loads rather than on one chain of dependent ones, and into eight sums of
+// Loads go out eight chunks at a time, the last ones too, so a thread waits on a few batches
+// of independent loads rather than on one chain of dependent ones (47 chunks of 1x1x6000x64
+// bf16 12.2 us with the last seven one after another, 9.6 so), and into eight sums of
 // their own: one chain over up to 512 chunks would round every term at the size of the
 // whole sum (f32 1x1x16000x64, 125 chunks: relative error 3.1e-7 in one chain, 2.0e-7 here).
 // An empty chunk (m = -inf, l = acc = 0) gets weight exp2(-inf) = 0.
@@ -266,20 +273,25 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float* __rest
   const bool valid = p >= 0 && p < max_len;
   const int used = valid ? min(nchunks, p / chunk + 1) : 0;
   const float* src = part + bh * nchunks * S;
+  const int full = used / G * G;
   float mx = -INFINITY;
-  int s0 = 0;
-  for (; s0 + G <= used; s0 += G) {
+  for (int s = 0; s < full; s += G) {
     float m[G];
 #pragma unroll
-    for (int j = 0; j < G; ++j) m[j] = src[(s0 + j) * S + D];
+    for (int j = 0; j < G; ++j) m[j] = src[(s + j) * S + D];
 #pragma unroll
     for (int j = 0; j < G; ++j) mx = fmaxf(mx, m[j]);
   }
-  for (; s0 < used; ++s0) mx = fmaxf(mx, src[s0 * S + D]);
+  if (full < used) {
+    float m[G];
+#pragma unroll
+    for (int j = 0; j < G; ++j) m[j] = src[min(full + j, used - 1) * S + D];
+#pragma unroll
+    for (int j = 0; j < G; ++j) mx = fmaxf(mx, m[j]);
+  }
   for (int e = threadIdx.x; e < D; e += blockDim.x) {
     float ls[G] = {}, as[G] = {};
-    int s = 0;
-    for (; s + G <= used; s += G) {
+    for (int s = 0; s < full; s += G) {
       float m[G], lv[G], av[G];
 #pragma unroll
       for (int j = 0; j < G; ++j) {
@@ -294,10 +306,21 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float* __rest
         as[j] += av[j] * w;
       }
     }
-    for (; s < used; ++s) {
-      const float w = exp2f(src[s * S + D] - mx);
-      ls[0] += src[s * S + D + 1] * w;
-      as[0] += src[s * S + e] * w;
+    if (full < used) {  // past the last chunk its own partial again, not added
+      float m[G], lv[G], av[G];
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const float* c = src + min(full + j, used - 1) * S;
+        m[j] = c[D];
+        lv[j] = c[D + 1];
+        av[j] = c[e];
+      }
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const float w = exp2f(m[j] - mx);
+        ls[j] += full + j < used ? lv[j] * w : 0.f;
+        as[j] += full + j < used ? av[j] * w : 0.f;
+      }
     }
 #pragma unroll
     for (int n = G / 2; n > 0; n /= 2)
@@ -310,8 +333,10 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const float* __rest
   }
 }
 
-int64_t chunks_for(int64_t b, int64_t h, int64_t max_len) {
+// No more chunks than a workspace of the smallest ones holds, for any row.
+int64_t chunks_for(int64_t b, int64_t h, int64_t max_len, int row_bytes = 0) {
   int64_t c = kChunkMin;
+  if (row_bytes && cdiv(max_len, c) * kRowBytesPerChunk > row_bytes) c *= 2;
   while (c < max_len && b * h * cdiv(max_len, c) > kGridTarget) c *= 2;
   return cdiv(max_len, c);
 }
@@ -321,7 +346,7 @@ int decode_launch(const void* q, const void* kn, const void* vn, void* kc, void*
                   int64_t B, int64_t H, int64_t L, float scale, void* ws, int64_t ws_bytes, int64_t new_stride,
                   hipStream_t st) {
   constexpr int kStep = kStepRows<T, D>;
-  int64_t nch = chunks_for(B, H, L);
+  int64_t nch = chunks_for(B, H, L, D * (int)sizeof(T));
   const bool one_group = nch > 1 && L <= 16 * 2 * kStep;
   const bool fits = ws && ws_bytes >= B * H * nch * (D + 2) * (int64_t)sizeof(float);
   if (one_group || (!fits && L <= kNoWorkspaceRows)) nch = 1;

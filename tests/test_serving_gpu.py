@@ -278,3 +278,22 @@ def test_decode_attention_sums_of_many_chunks(dev):
         ref = (p.unsqueeze(-1) * vc.double()).sum(2)
         err.append(float((out.double() - ref).norm() / ref.norm()))
     assert np.mean(err) <= 2.6e-7, np.mean(err)
+
+
+@pytest.mark.parametrize("L,d,dtype", [
+    (4096, 64, torch.bfloat16), (4097, 64, torch.bfloat16),  # the last in chunks of 128 rows, the first in 256
+    (8192, 64, torch.float32), (8193, 64, torch.float32),
+    (2500, 256, torch.bfloat16),
+])
+def test_decode_attention_of_every_chunk_count(dev, L, d, dtype):
+    """Positions in each of the first 18 chunks and the last: whole and ragged batches of the second pass, and
+    whole caches on both sides of the chunks' rule, against the restatement in float64."""
+    pos = [128 * i + (7 * i) % 128 for i in range(18)] + [L - 1, L - 2, 127, 128]
+    q, kn, vn, kc, vc = _case(dev, 1, 2, L, d, dtype, L)
+    for p in pos:
+        k, v = kc.clone(), vc.clone()
+        out = decode_attention(q, kn, vn, k, v, torch.tensor([p], dtype=torch.int32, device=dev))
+        k, v = (t[0, :, : p + 1].double() for t in (k, v))
+        ref = (torch.softmax((k * q[0].double().unsqueeze(1)).sum(-1) * d**-0.5, -1).unsqueeze(-1) * v).sum(1)
+        # one rounding to bf16 (half an ulp, 2^-9 of the value); f32 sums as in the cases above
+        assert ((out[0].double() - ref).abs() <= (2.0**-8 if dtype == torch.bfloat16 else 0.0) * ref.abs() + 1e-5).all(), p
