@@ -172,10 +172,18 @@ def _one_kernel_embedding(tok, pe, token, pos, dtype) -> bool:
 
 
 def _few_rows_head(y, emb) -> bool:
-    """Whether the tied head runs on the few-rows kernel, which reads the embedding as it is: up to
-    64 rows of bf16 and 2^24 weights (beyond those the library product is level or faster)."""
-    return y.dtype == torch.bfloat16 and emb.dtype in (torch.float32, torch.bfloat16) and y.shape[0] <= 64 \
-        and emb.numel() <= 1 << 24
+    """Whether the tied head's bf16 rows run on the few-rows kernel, which reads the embedding as it is. us
+    on one MI355X, that kernel / a bf16 copy of a float embedding and the library's product, V x d weights:
+    float   8 rows, 1000 x 512 5.7 / 8.4   32, 8192 x 2048 19.4 / 25.5   64, 8192 x 1024 15.6 / 19.3
+            40, 8192 x 2048 27.2 / 26.4    64, 32768 x 512 28.2 / 26.3
+    bf16    8, 8192 x 512 5.1 / 5.4        32, 1000 x 512 5.6 / 6.2      64, 256 x 512 7.3 / 10.0
+            64, 8192 x 512 8.0 / 7.2       8, 1000 x 1024 6.2 / 5.6      8, 4096 x 4096 11.2 / 9.8"""
+    rows, weights = y.shape[0], emb.numel()
+    if y.dtype != torch.bfloat16 or rows > 64:
+        return False
+    if emb.dtype == torch.float32:
+        return weights <= 1 << (24 if rows <= 32 else 23)
+    return emb.dtype == torch.bfloat16 and emb.shape[1] <= 512 and weights <= 1 << (22 if rows <= 32 else 17)
 
 
 # The serving engine: captured prefill per bucket, one captured decode step.

@@ -113,3 +113,18 @@ def test_one_kernel_embedding_leaves_other_devices_to_indexing():
         case = [tok, pe, t, p]
         case[at] = case[at].to("meta")
         assert not _one_kernel_embedding(*case, torch.bfloat16)
+
+
+def test_few_rows_head_keeps_to_where_it_is_faster():
+    """Every side of the rule's lines, as measured: a float embedding's copy costs more than a bf16 one's."""
+    from ferrite.serving.engine import _few_rows_head
+
+    f32, bf16 = torch.float32, torch.bfloat16
+    cases = [(8, 1000, 512, f32, True), (32, 8192, 2048, f32, True), (33, 8192, 2048, f32, False),
+             (64, 8192, 1024, f32, True), (65, 256, 256, f32, False), (1, 8193, 2048, f32, False),
+             (32, 8192, 512, bf16, True), (33, 8192, 512, bf16, False), (8, 1000, 1024, bf16, False),
+             (64, 256, 512, bf16, True), (8, 32768, 512, bf16, False), (8, 256, 256, torch.float16, False)]
+    for rows, v, d, dtype, takes in cases:
+        emb = torch.empty(v, d, dtype=dtype, device="meta")
+        assert _few_rows_head(torch.empty(rows, d, dtype=bf16, device="meta"), emb) == takes, (rows, v, d, dtype)
+        assert not _few_rows_head(torch.empty(rows, d, dtype=f32, device="meta"), emb)
