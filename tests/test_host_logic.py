@@ -60,22 +60,26 @@ def test_internal_entry_points_match_their_header():
     assert declared == set(_hip.INTERNAL) and not declared & set(_hip.SIGNATURES)
 
 
+def _on_gpu(*shape, dtype=None):
+    """What the rules ask of a tensor on a GPU."""
+    from types import SimpleNamespace
+
+    import torch
+
+    return SimpleNamespace(shape=shape, ndim=len(shape), dtype=dtype or torch.float32, device="cuda:0", is_cuda=True,
+                           numel=lambda: int(torch.Size(shape).numel()))
+
+
 def test_embedding_rules_stay_within_a_launch():
     """A block of 256 threads per token and position, and under 2^32 threads along a grid's x: the rules
     leave more to torch's indexing, and the entry points refuse it before a launch."""
-    from types import SimpleNamespace
-
     import torch
 
     from ferrite import _hip
     from ferrite.model import gpt
     from ferrite.serving import engine
 
-    def tensor(*shape, dtype=torch.float32):
-        return SimpleNamespace(shape=shape, ndim=len(shape), dtype=dtype, device="cuda:0", is_cuda=True,
-                               numel=lambda: int(torch.Size(shape).numel()))
-
-    i64, bf16, most = torch.int64, torch.bfloat16, (1 << 24) - 1
+    tensor, i64, bf16, most = _on_gpu, torch.int64, torch.bfloat16, (1 << 24) - 1
     for n, takes in ((most, True), (most + 1, False)):
         assert gpt._one_kernel_embedding(tensor(256, 8), tensor(4, 8), tensor(n, 1, dtype=i64), bf16) == takes
         assert gpt._one_kernel_embedding(tensor(256, 8), tensor(n, 8), tensor(3, 4, dtype=i64), bf16) == takes
@@ -84,3 +88,17 @@ def test_embedding_rules_stay_within_a_launch():
         assert _hip.lib().ferrite_internal_embed(None, None, None, None, None, n, 8, 256, 4, 4, 0, 0, None) == 1
         assert ("null" if takes else "sizes") in _hip.last_error()
         assert (_hip.lib().ferrite_internal_embed_bwd_workspace(12, 4, 8, 256, n) > 0) == takes
+
+
+def test_training_embedding_keeps_to_where_it_is_faster():
+    """Every side of the rule's lines: vocabularies past 512 tokens with wide rows stay with torch's sorted sums."""
+    import torch
+
+    from ferrite.model import gpt
+
+    for tokens, dim, vocab, takes in [(16384, 512, 1000, True), (16384, 513, 1000, False), (16384, 513, 512, True),
+                                      (8192, 1024, 1024, True), (2048, 2048, 1024, True), (4096, 2048, 1024, False), (131072, 256, 1024, True),
+                                      (131072, 4096, 512, True), (4, 64, 1025, False)]:
+        got = gpt._one_kernel_embedding(_on_gpu(vocab, dim), _on_gpu(8, dim), _on_gpu(tokens // 4, 4, dtype=torch.int64),
+                                        torch.bfloat16)
+        assert got == takes, (tokens, dim, vocab)
