@@ -293,15 +293,16 @@ def _one_kernel_embedding(tok, pe, tokens, dtype) -> bool:
     holds) and plain indices; a table row per position; a block per token and position, in one launch
     under 2^32 threads. Over 512 tokens a wave's table holds 16 columns, so that every row is loaded
     four times: there up to 256 columns, or 2^23 elements of output (2^22 in rows of over 1024). us
-    forward and backward on one MI355X, torch's indexing / the kernels: 16384 x 512 over 256 tokens 182 / 64, over 512 144 / 75, over
-    1000 144 / 114; 1024 x 512 over 1000 139 / 63; 128 x 128 over 256 132 / 64. bf16 tables: 65536 x 4096
+    forward and backward on one MI355X, torch's indexing / the kernels: 16384 x 512 over 256 tokens
+    182 / 64, over 512 144 / 75, over 1000 144 / 114; 1024 x 512 over 1000 139 / 63; 128 x 128 over 256 132 / 64. bf16 tables: 65536 x 4096
     over 512 2018 / 1533; over 1024 16384 x 512 130 / 116, 131072 x 256 437 / 368, past the line
     16384 x 768 133 / 164, 4096 x 2048 93 / 119."""
     floats = (torch.float32, torch.bfloat16)
     return (tok.is_cuda and tok.device == pe.device == tokens.device and tok.dtype == pe.dtype
             and tok.dtype in floats and dtype in floats and tok.ndim == pe.ndim == 2
             and tok.shape[1] == pe.shape[1] and 0 < tok.shape[0] <= 1024 and 0 < tok.shape[1] <= 1 << 20
-            and (tok.shape[0] <= 512 or tok.shape[1] <= 256 or tokens.numel() * tok.shape[1] <= 1 << (23 if tok.shape[1] <= 1024 else 22))
+            and (tok.shape[0] <= 512 or tok.shape[1] <= 256
+                 or tokens.numel() * tok.shape[1] <= 1 << (23 if tok.shape[1] <= 1024 else 22))
             and tokens.ndim == 2 and tokens.dtype in (torch.int64, torch.int32)
             and 0 < tokens.numel() < 1 << 24 and tokens.shape[1] <= pe.shape[0] < 1 << 24)
 
