@@ -4142,7 +4142,7 @@ int fwd_launch(const void* q, const void* k, const void* v, void* o, float* lse,
   const int64_t bh = s.b * s.h;
   if (nq * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_fwd: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (sched::f32_shared_sweeps(nq * bh, causal, D <= 64, cu_count(stream)))
+    if (sched::f32_shared_sweeps(sched::F32Pass::kFwd, bh, s.sq, s.sk, s.d, causal, cu_count(stream)))
       return f32_attn_fwd(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                           static_cast<float*>(o), lse, {bh, s.sq, s.sk, s.d, causal}, scale, stream);
   }
@@ -4270,7 +4270,7 @@ int dq_launch(const void* q, const void* k, const void* v, const void* dout, con
   const int64_t bh = s.b * s.h;
   if (nq * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_bwd_dq: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (sched::f32_shared_sweeps(nq * bh, causal, D <= 64, cu_count(stream)))
+    if (sched::f32_shared_sweeps(sched::F32Pass::kDq, bh, s.sq, s.sk, s.d, causal, cu_count(stream)))
       return f32_attn_dq(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                          static_cast<const float*>(dout), lse, delta, static_cast<float*>(dq),
                          {bh, s.sq, s.sk, s.d, causal}, scale, stream);
@@ -4351,7 +4351,7 @@ int dkv_launch(const void* q, const void* k, const void* v, const void* dout, co
   const int64_t bh = s.b * s.h;
   if (nk * bh > 0x7fffffff) return fail(FERRITE_ERR_INVALID_ARGUMENT, "ferrite_hip_attn_bwd_dkv: grid too large");
   if constexpr (sizeof(T) == 4 && AL && D <= 128) {
-    if (sched::f32_shared_sweeps(nk * bh, causal, false, cu_count(stream)))
+    if (sched::f32_shared_sweeps(sched::F32Pass::kDkv, bh, s.sk, s.sq, s.d, causal, cu_count(stream)))
       return f32_attn_dkv(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                           static_cast<const float*>(dout), lse, delta, static_cast<float*>(dk),
                           static_cast<float*>(dv), {bh, s.sq, s.sk, s.d, causal}, scale, stream);

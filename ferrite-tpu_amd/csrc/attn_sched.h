@@ -142,20 +142,38 @@ FERRITE_SCHED int fwd_split_cut(long long bh, long long S, int cus) { return spl
 // `per_cu` workgroups per CU: when all of them are resident at once.
 FERRITE_SCHED bool resident(long long grid, int per_cu, int cus) { return grid <= (long long)per_cu * cus; }
 
-// Whether an f32 pass takes the kernels whose waves share a sweep (attn_f32.hip) rather than those
-// with 128 rows a workgroup, given the latter's grid. Theirs is the better rate once they fill the
-// chip evenly, their waves sharing tiles through LDS: from a workgroup per CU on without a mask,
-// from two with one (whose sweeps differ in length). us on one MI355X, 128 rows / shared sweeps:
-//   2x8x1024x64 causal (128 workgroups): forward 82 / 34, dQ 119 / 50, dK/dV 155 / 62
-//   1x8x4096x64 causal (256): 308 / 158, 459 / 235, 606 / 356
-//   2x8x1024x128 (128): 137 / 92, 211 / 126, 293 / 164
-//   8x16x256x64 (256): 25 / 29, 35 / 44, 47 / 62
-//   4x16x1024x128 causal (512): 193 / 212, 243 / 300, 341 / 395
-//   4x16x1024x64 causal (512): 113 / 86, 166 / 133, 208 / 222
-// With two waves per SIMD (the forward and dQ up to head dim 64) a causal grid is theirs while their
-// four workgroups of 32 rows for one of 128, of 256 threads each, stay under a launch's 2^32 threads.
-FERRITE_SCHED bool f32_shared_sweeps(long long workgroups, int causal, bool two_waves, long long cus) {
-  return workgroups < (causal ? 2 : 1) * cus || (causal && two_waves && workgroups < 1LL << 22);
+// Whether an f32 pass takes the kernels whose waves share a sweep (attn_f32.hip: a workgroup per
+// 32 rows) rather than those whose waves each sweep alone (128 rows), for `bh` heads of `own` rows
+// (queries; keys in dK/dV) that sweep `sweep` of the other side. Never past a workgroup per CU of
+// the latter without a mask, or two with one (the sweeps of a causal grid differ in length; the
+// forward and dQ up to head dim 64, with two waves per SIMD, go on): from there those fill the chip, and
+// share tiles through LDS. Within, by their times in products of one 32-row tile (n of them in a
+// sweep): a shared sweep takes n / 4 in each of four waves, and the start and end of its
+// workgroup as long as two more; alone, n, n + 2 with the ends, or 5 / 4 of that with two workgroups
+// on a CU. A causal grid of several rounds averages 5/8 of a sweep. us on one MI355X, 128 rows /
+// shared sweeps, where that line lies (forward, dQ or dK/dV of heads x own x sweep x head dim):
+//   taken:  forward causal 16x1024x1024x64 81 / 33   dQ 24x512x128x128 36 / 34      dK/dV causal 64x256x256x64 45 / 28
+//   left:   dK/dV 24x1024x16x64 13.5 / 25            dQ 24x1024x64x128 25 / 43      forward causal 200x256x256x128 56 / 87
+// Past one round, the forward and dQ up to head dim 64 still win with long sweeps: causal up to two
+// workgroups per CU from 12 tiles on (64x1024x1024x64 108 / 87; 300x768x768x64 216 / 257 stays), any
+// grid from 64 on (40x640x8192x64 620 / 511). One tile leaves three of the waves idle (dQ causal
+// 200x32x32x128 12.5 / 14.7). Up to head dim 32 the shared sweeps win nearly everywhere
+// (24x1024x1024 causal 82 / 24). Over 6810 measured shapes eight taken are over 4% slower than left,
+// one over 11% (dQ 200x128x16x32 9.1 / 12.0).
+// Their four workgroups for one, of 256 threads each, stay under a launch's 2^32 threads.
+enum class F32Pass { kFwd, kDq, kDkv };
+FERRITE_SCHED bool f32_shared_sweeps(F32Pass pass, long long bh, long long own, long long sweep, long long d, int causal,
+                                     long long cus) {
+  const bool dkv = pass == F32Pass::kDkv, two_waves = d <= 64 && !dkv;
+  const long long apart = bh * ((own + 127) / 128), n = (sweep + 31) / 32;
+  if (apart >= 1LL << 22 || !(apart < (causal ? 2 : 1) * cus || (causal && two_waves))) return false;
+  if (d <= 32) return true;
+  if (n == 1 && own < 128 && (pass == F32Pass::kDq || (pass == F32Pass::kFwd && d > 64))) return false;
+  if (two_waves && ((causal && n >= 12 && apart <= 2 * cus) || n >= 64)) return true;
+  const long long rounds = (bh * ((own + 31) / 32) + cus - 1) / cus;
+  const long long shared_time = rounds * ((causal && rounds > 1 ? 5 : 8) * n + 64);  // in eighths of a quarter tile
+  const long long apart_time = (n + 2) * (apart <= cus ? 32 : 40 * ((apart + 2 * cus - 1) / (2 * cus)));
+  return shared_time <= apart_time;
 }
 
 // ---- rings -------------------------------------------------------------------

@@ -622,20 +622,41 @@ static void check_wide(int bh, int S, int D) {
 }
 
 // The f32 kernels with shared sweeps (f32_shared_sweeps): a workgroup of 256 threads per 32 rows, under 2^32
-// threads along x for every grid the rule gives them.
-static void check_f32_grids() {
-  for (int causal : {0, 1})
-    for (bool two_waves : {false, true})
-      for (long long nq : {1LL, 3LL, 64LL})
-        for (long long bh = 1; nq * bh < 1LL << 24; bh = bh * 3 / 2 + 1)
-          for (long long b : {bh, (1LL << 22) / nq, (1LL << 22) / nq - 1}) {
-            const long long S = 128 * nq;
-            if (f32_shared_sweeps(nq * b, causal, two_waves, kCus) && (S + 31) / 32 * b * 256 >= 1LL << 32)
-              fail("f32: the grid of " + std::to_string(b) + " heads of " + std::to_string(S) + " rows is too large");
-          }
-  if (!f32_shared_sweeps(256, 1, false, kCus) || !f32_shared_sweeps(1 << 20, 1, true, kCus) ||
-      f32_shared_sweeps(256, 0, true, kCus) || f32_shared_sweeps(512, 1, false, kCus))
-    fail("f32: the sweeps are shared on the wrong grids");
+// threads along x for every grid the rule gives them; and both sides of the rule's lines, as measured.
+static void check_f32_rule() {
+  const F32Pass passes[] = {F32Pass::kFwd, F32Pass::kDq, F32Pass::kDkv};
+  for (F32Pass pass : passes)
+    for (int causal : {0, 1})
+      for (long long d : {32LL, 64LL, 128LL})
+        for (long long nq : {1LL, 3LL, 64LL})
+          for (long long bh = 1; nq * bh < 1LL << 24; bh = bh * 3 / 2 + 1)
+            for (long long b : {bh, (1LL << 22) / nq, (1LL << 22) / nq - 1}) {
+              const long long S = 128 * nq;
+              if (f32_shared_sweeps(pass, b, S, S, d, causal, kCus) && (S + 31) / 32 * b * 256 >= 1LL << 32)
+                fail("f32: the grid of " + std::to_string(b) + " heads of " + std::to_string(S) + " rows is too large");
+            }
+  struct Case {
+    F32Pass pass;
+    long long bh, own, sweep, d;
+    int causal;
+    bool shared;
+  };
+  const Case cases[] = {
+      {F32Pass::kFwd, 16, 1024, 1024, 64, 1, true},   {F32Pass::kDkv, 16, 1024, 1024, 64, 1, true},
+      {F32Pass::kFwd, 24, 512, 64, 128, 0, false},    {F32Pass::kFwd, 24, 512, 128, 128, 0, true},
+      {F32Pass::kDkv, 30, 1024, 26, 48, 0, false},    {F32Pass::kDq, 24, 1024, 64, 128, 0, false},
+      {F32Pass::kFwd, 200, 256, 256, 128, 1, false},  {F32Pass::kDq, 16, 1761, 384, 80, 0, false},
+      {F32Pass::kFwd, 64, 1024, 1024, 64, 1, true},   {F32Pass::kDkv, 64, 1024, 1024, 64, 1, false},
+      {F32Pass::kFwd, 300, 768, 768, 64, 1, false},   {F32Pass::kFwd, 300, 2048, 2048, 64, 1, true},
+      {F32Pass::kFwd, 40, 640, 8192, 64, 0, true},    {F32Pass::kFwd, 52, 640, 8192, 64, 0, false},
+      {F32Pass::kDq, 8, 32, 32, 128, 1, false},       {F32Pass::kDkv, 8, 32, 32, 128, 1, true},
+      {F32Pass::kFwd, 5000, 512, 512, 32, 1, true},   {F32Pass::kDkv, 5000, 512, 512, 32, 1, false},
+      {F32Pass::kFwd, 130, 256, 512, 64, 0, false},
+  };
+  for (const Case& c : cases)
+    if (f32_shared_sweeps(c.pass, c.bh, c.own, c.sweep, c.d, c.causal, kCus) != c.shared)
+      fail("f32: " + std::to_string(c.bh) + " heads of " + std::to_string(c.own) + " over " + std::to_string(c.sweep) +
+           " at head dim " + std::to_string(c.d) + " on the slower kernels");
 }
 
 int main() {
@@ -644,7 +665,7 @@ int main() {
   lengths.push_back(8192);
   const int bhs[] = {1, 3, 8, 64};
   int launches = 0;
-  check_f32_grids();
+  check_f32_rule();
   for (int bh : bhs)
     for (int S : lengths) {
       // The forward's launch choices (fwd_launch): D = 128 one 8-wave workgroup per CU; D <= 64 the
