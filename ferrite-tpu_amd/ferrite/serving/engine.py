@@ -177,13 +177,14 @@ def _few_rows_head(y, emb) -> bool:
     float   8 rows, 1000 x 512 5.7 / 8.4   32, 8192 x 2048 19.4 / 25.5   64, 8192 x 1024 15.6 / 19.3
             40, 8192 x 2048 27.2 / 26.4    64, 32768 x 512 28.2 / 26.3
     bf16    8, 8192 x 512 5.1 / 5.4        32, 1000 x 512 5.6 / 6.2      64, 256 x 512 7.3 / 10.0
-            64, 8192 x 512 8.0 / 7.2       8, 1000 x 1024 6.2 / 5.6      8, 4096 x 4096 11.2 / 9.8"""
+            64, 8192 x 512 8.0 / 7.2       8, 1000 x 1024 6.2 / 5.6      32, 300 x 129 6.5 / 5.7"""
     rows, weights = y.shape[0], emb.numel()
     if y.dtype != torch.bfloat16 or rows > 64:
         return False
     if emb.dtype == torch.float32:
         return weights <= 1 << (24 if rows <= 32 else 23)
-    return emb.dtype == torch.bfloat16 and emb.shape[1] <= 512 and weights <= 1 << (22 if rows <= 32 else 17)
+    d = emb.shape[1]
+    return emb.dtype == torch.bfloat16 and d <= 512 and d % 8 == 0 and weights <= 1 << (22 if rows <= 32 else 17)
 
 
 # The serving engine: captured prefill per bucket, one captured decode step.
