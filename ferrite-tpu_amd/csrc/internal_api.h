@@ -20,6 +20,12 @@ extern "C" {
  */
 int64_t ferrite_internal_matmul_ragged_workspace(const void* x, const void* y, int64_t m, int64_t n, int64_t k,
                                                  int x_t, int y_t);
+/*
+ * 1 where that is the faster one, 0 where ferrite_hip_matmul_ex's own choice on untransposed operands is
+ * (transposed ones copied first).
+ */
+int ferrite_internal_matmul_ragged_better(const void* x, const void* y, int64_t m, int64_t n, int64_t k, int x_t,
+                                          int y_t);
 int ferrite_internal_matmul_ragged(const void* x, const void* y, void* out, int64_t m, int64_t n, int64_t k, int x_t,
                                    int y_t, int out_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 

@@ -1190,6 +1190,25 @@ bool rag_ok(int64_t m, int64_t n, int64_t k, bool xt, bool yt) {
          k * (n + 8) / 8 < 0x3fffffff;
 }
 
+// Whether the ragged kernel beats gemm_kernel, which loads unaligned operands by elements in one launch (and
+// has a transposed one copied first). Where nothing is packed it does from pick_bm's quarter of the CUs'
+// worth of 256 x 256 tiles on, or with a split K: gemm_kernel's smaller tiles spread few outputs over
+// more CUs. Where y is packed, that has to be earned back over more than a k-step or two; x alone is as
+// cheap to pack as to load by elements but for narrow outputs.
+// us on one MI355X, gemm_kernel / packing and the ragged kernel (M x K x N):
+//   aligned rows: 1030 x 520 x 264 14 / 16   1030 x 1000 x 264 20 / 23   1030 x 1096 x 264 (split) 21 / 19
+//   4100 x 136 x 520 (51 tiles) 9.6 / 12     8190 x 520 x 264 (64 tiles) 22 / 16
+//   y packed: 2050 x 33 x 30 8.2 / 13   1030 x 64 x 1030 14 / 14   2050 x 100 x 30 11 / 14
+//   2050 x 136 x 30 13 / 15, x 66 15 / 15   4100 x 200 x 130 23 / 17     x alone: 520 x 20 x 264 12 / 10, x 8 8.3 / 9.9
+//   y copied or packed: 1030 x 20 x 30 11 / 13, x 66 11 / 13, x 130 14 / 14
+bool rag_better(const RagPlan& p, int64_t M, int64_t N, int64_t K, bool copies, int64_t cus) {
+  const int64_t tiles = cdiv(M, (int64_t)128) * cdiv(N, (int64_t)128), steps = cdiv(K, (int64_t)Gemm2::BK);
+  if (copies) return steps > 1 || N > 128 || N % 8 == 0 || !p.pack_y;
+  if (p.pack_y) return steps > (N <= 64 ? 3 : 2) || steps * 2 * tiles > cus;
+  if (p.pack_x) return steps > 1 || N > 64;
+  return p.slices > 1 || cdiv(M, (int64_t)Gemm2::BM) * cdiv(N, (int64_t)Gemm2::BN) >= cus / 4;
+}
+
 template <typename TO, bool XT, bool YT>
 int launch_gemm_rag_t(const bf16* x, const bf16* y, TO* out, int64_t M, int64_t N, int64_t K, const RagPlan& p,
                       char* ws, hipStream_t stream) {
@@ -1269,6 +1288,16 @@ extern "C" int64_t ferrite_internal_matmul_ragged_workspace(const void* x, const
   return ferrite::rag_plan(x, y, m, n, k, xt, yt, ferrite::cu_count_of(-1)).bytes;
 }
 
+extern "C" int ferrite_internal_matmul_ragged_better(const void* x, const void* y, int64_t m, int64_t n, int64_t k,
+                                                     int x_t, int y_t) {
+  using namespace ferrite;
+  if (m < 1 || n < 1 || k < 1) return 0;
+  const bool xt = x_t != 0, yt = y_t != 0;
+  if (!xt && skinny_ok(m, n, k)) return 1;
+  const int64_t cus = cu_count_of(-1);
+  return rag_ok(m, n, k, xt, yt) && rag_better(rag_plan(x, y, m, n, k, xt, yt, cus), m, n, k, xt || yt, cus);
+}
+
 extern "C" int ferrite_internal_matmul_ragged(const void* x, const void* y, void* out, int64_t m, int64_t n, int64_t k,
                                               int x_t, int y_t, int out_dtype, void* workspace,
                                               int64_t workspace_bytes, void* stream) {
@@ -1340,8 +1369,8 @@ extern "C" int ferrite_hip_matmul_ex(const void* x, const void* y, void* out, in
   if (in_dtype == FERRITE_BF16 && !xt && !yt && rag_ok(m, n, k, xt, yt)) {
     // Aligned rows and a K that is no whole number of 64-deep steps: nothing to pack.
     RagPlan p = rag_plan(x, y, m, n, k, xt, yt, cu_count(s));
-    if (!p.pack_x && !p.pack_y) {
-      if (!workspace || workspace_bytes < p.bytes || (reinterpret_cast<uintptr_t>(workspace) & 15)) p.slices = 1;
+    if (!workspace || workspace_bytes < p.bytes || (reinterpret_cast<uintptr_t>(workspace) & 15)) p.slices = 1;
+    if (!p.pack_x && !p.pack_y && rag_better(p, m, n, k, false, cu_count(s))) {
       if (out_dtype == FERRITE_BF16) return launch_gemm_rag<bf16>(x, y, out, m, n, k, xt, yt, p, workspace, s);
       return launch_gemm_rag<float>(x, y, out, m, n, k, xt, yt, p, workspace, s);
     }
@@ -1351,8 +1380,8 @@ extern "C" int ferrite_hip_matmul_ex(const void* x, const void* y, void* out, in
                 "ferrite_hip_matmul: transposed operands need bf16, K % 64 == 0, N % 8 == 0, M % 8 == 0 for a "
                 "transposed x, and 16-byte aligned pointers");
   if (in_dtype == FERRITE_BF16) {
-    // Shapes the DMA kernel does not read in place (unaligned rows or pointers), with no
-    // workspace to pack them into: four waves of 64 x 64 outputs per 128 x 128 tile (256 x 256 tiles spilled 48 bytes per lane).
+    // What the kernels above leave, and unaligned rows with no workspace to pack them into: four
+    // waves of 64 x 64 outputs per 128 x 128 tile (256 x 256 tiles spilled 48 bytes per lane).
     if (out_dtype == FERRITE_BF16) return launch_gemm<bf16, bf16, 128, 128, 64, 2, 2>(x, y, out, m, n, k, s);
     return launch_gemm<bf16, float, 128, 128, 64, 2, 2>(x, y, out, m, n, k, s);
   }

@@ -269,8 +269,8 @@ Tensor transposed(const Tensor& t, int64_t rows, int64_t cols) { return t.view({
 
 // op(x) @ op(y) of m x k and k x n matrices in `shape` (m n elements). x holds the m x k matrix, or
 // its transpose when x_t; y the k x n one, or its transpose when y_t. bf16 operands of other
-// sizes or alignment than the kernel reads in place go through ferrite_internal_matmul_ragged; a
-// transposed f32 operand is transposed into a copy first.
+// sizes or alignment than the kernel reads in place go through ferrite_internal_matmul_ragged where
+// it is the faster one; a transposed f32 operand is transposed into a copy first.
 Tensor mm(const Tensor& x0, const Tensor& y0, int64_t m, int64_t n, int64_t k, bool x_t, bool y_t,
           at::ScalarType out_dtype, at::IntArrayRef shape) {
   // Mixed operand dtypes are promoted as jnp.dot would; widening bf16 to f32 is exact.
@@ -278,12 +278,14 @@ Tensor mm(const Tensor& x0, const Tensor& y0, int64_t m, int64_t n, int64_t k, b
   Tensor x = x0.to(work).contiguous(), y = y0.to(work).contiguous();
   const auto kernel_out = out_dtype == at::kFloat || out_dtype == at::kBFloat16 ? out_dtype : at::kFloat;
   Tensor out = at::empty(shape, x.options().dtype(kernel_out));
+  x_t = x_t && m > 1;  // a column of single elements is a row
+  y_t = y_t && k > 1;
   if (m && n && k == 0) out.zero_();
   if (m && n && k) {
     const bool direct = in_place(work, m, n, k, x_t, x, y, out);
-    const int64_t rag = work == at::kBFloat16 && !direct
-                            ? ferrite_internal_matmul_ragged_workspace(ptr(x), ptr(y), m, n, k, x_t, y_t)
-                            : -1;
+    const bool ragged = work == at::kBFloat16 && !direct &&
+                        ferrite_internal_matmul_ragged_better(ptr(x), ptr(y), m, n, k, x_t, y_t);
+    const int64_t rag = ragged ? ferrite_internal_matmul_ragged_workspace(ptr(x), ptr(y), m, n, k, x_t, y_t) : -1;
     if (rag >= 0) {
       const Tensor ws = bytes_on(rag, x);
       check(ferrite_internal_matmul_ragged(ptr(x), ptr(y), ptr(out), m, n, k, x_t, y_t, code(kernel_out), ptr(ws), rag,

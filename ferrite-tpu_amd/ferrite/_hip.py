@@ -121,6 +121,7 @@ SIGNATURES: dict[str, tuple] = {
 # Entry points for this package alone; must match csrc/internal_api.h.
 INTERNAL: dict[str, tuple] = {
     "ferrite_internal_matmul_ragged_workspace": (_c_i64, [_vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int]),
+    "ferrite_internal_matmul_ragged_better": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int]),
     "ferrite_internal_matmul_ragged": (
         _c_int,
         [_vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _vp, _c_i64, _vp],

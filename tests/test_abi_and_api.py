@@ -262,3 +262,22 @@ def test_cross_entropy_grad_takes_two_dims(shape):
 
     with pytest.raises(ValueError, match="logits"):
         cross_entropy_grad(torch.zeros(shape), torch.zeros(2, dtype=torch.long), torch.zeros(2), torch.ones(()), 1.0)
+
+
+def test_ragged_products_keep_to_where_they_are_faster():
+    """Both sides of the lines between packing and the kernel that loads by elements, as measured, from
+    stand-in addresses: 256 CUs, aligned operands unless `at` says otherwise."""
+    a = 1 << 12
+    for m, k, n, at, layout, takes in [
+        (1030, 520, 264, a, (0, 0), 0), (1030, 1096, 264, a, (0, 0), 1), (8190, 520, 264, a, (0, 0), 1),  # nothing to pack
+        (65, 8, 8, a, (0, 0), 0), (64, 8, 8, a, (0, 0), 1),                                             # few rows
+        (2050, 33, 30, a, (0, 0), 0), (1030, 64, 1030, a, (0, 0), 0), (2050, 64, 1030, a, (0, 0), 1),     # y: one step
+        (2050, 100, 30, a, (0, 0), 0), (1030, 100, 1030, a, (0, 0), 1), (2050, 136, 30, a, (0, 0), 0),    # two, three
+        (2050, 136, 66, a, (0, 0), 1), (2050, 200, 30, a, (0, 0), 1),
+        (520, 20, 264, a, (0, 0), 1), (520, 20, 8, a, (0, 0), 0), (520, 65, 8, a, (0, 0), 1),             # x alone
+        (1030, 64, 264, a + 2, (0, 0), 0), (1030, 136, 264, a + 2, (0, 0), 1),                          # y off its alignment
+        (1030, 20, 30, a, (0, 1), 0), (1030, 20, 130, a, (0, 1), 1), (1030, 20, 30, a, (1, 0), 0),        # a copy
+        (1030, 65, 30, a, (1, 0), 1), (4100, 136, 520, a, (0, 0), 0), (2050, 136, 2056, a, (0, 0), 1),
+    ]:
+        got = _hip.lib().ferrite_internal_matmul_ragged_better(a, at, m, n, k, *layout)
+        assert got == takes, (m, k, n, at, layout)
