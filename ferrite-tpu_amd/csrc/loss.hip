@@ -178,11 +178,15 @@ __global__ __launch_bounds__(kCeThreads) void ce_bwd_kernel(const float* __restr
   for (int64_t j = sp.tail + t; j < V; j += T) gr[j] = Elem<TO>::from_f32(one(x[j], j));
 }
 
-// Forward rows up to here take one wave each, four to a workgroup: a workgroup's merge costs
-// more than it saves (8192 x 2048 15.6 us on four waves, 10.8 on one; 8192 x 4096 20.9 on four).
-// The backward, which merges nothing, takes one up to 512 (16384 x 256: 6.7 us, 10.8 on four)
-// and two up to here (8192 x 1000 12.6 us, 13.9 on one, 13.2 on four).
-constexpr int64_t kShortRow = 2048;
+// Waves per row. Many short rows take one each, four to a workgroup: a workgroup's merge costs more than it
+// saves (forward, four waves / one: 4096 x 2048 12.7 / 9.4 us, 16384 x 1000 30 / 20, 65536 x 512 91 / 37; up to
+// 512 columns at any number of rows, 64 x 512 5.0 / 4.9), but few rows leave most CUs idle and wait
+// for their chains (64 x 1000 5.1 / 6.4, 512 x 2000 6.0 / 8.6, 1024 x 700 5.5 / 6.3). The backward, which
+// merges nothing, takes one up to 512 columns (16384 x 256 12.1 / 8.1) and two of many rows up to
+// 1536 (four / two: 4096 x 700 8.1 / 7.4; 512 x 2000 4.9 / 6.6, 4096 x 2000 13.6 / 15.4).
+constexpr int64_t kOneWave = 512, kManyRows = 2048;
+bool one_wave_fwd(int64_t n, int64_t v) { return v <= kOneWave || (n > kManyRows && v <= 2048); }
+bool two_waves_bwd(int64_t n, int64_t v) { return n > kManyRows && v <= 1536; }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -203,7 +207,7 @@ extern "C" int ferrite_hip_cross_entropy_fwd(const float* logits, const int64_t*
     hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(n, (int64_t)per_block)), dim3(kCeThreads), 0, s, logits, targets, loss,
                        lse, n, v);
   };
-  if (v <= kShortRow)
+  if (one_wave_fwd(n, v))
     vec ? go(ce_fwd_kernel<true, 1>, 4) : go(ce_fwd_kernel<false, 1>, 4);
   else
     vec ? go(ce_fwd_kernel<true, 4>, 1) : go(ce_fwd_kernel<false, 4>, 1);
@@ -229,9 +233,9 @@ extern "C" int ferrite_hip_cross_entropy_bwd(const float* logits, const int64_t*
   };
   auto rows = [&](auto* g) {
     typedef std::remove_pointer_t<decltype(g)> TO;
-    if (v <= 512)
+    if (v <= kOneWave)
       vec ? go(ce_bwd_kernel<TO, true, 1>, 4, g) : go(ce_bwd_kernel<TO, false, 1>, 4, g);
-    else if (v <= kShortRow)
+    else if (two_waves_bwd(n, v))
       vec ? go(ce_bwd_kernel<TO, true, 2>, 2, g) : go(ce_bwd_kernel<TO, false, 2>, 2, g);
     else
       vec ? go(ce_bwd_kernel<TO, true, 4>, 1, g) : go(ce_bwd_kernel<TO, false, 4>, 1, g);

@@ -82,8 +82,9 @@ def test_validation(dev):
 
 @pytest.mark.parametrize("n,v", [
     (3, 1), (70, 3), (7, 33),            # rows inside one 128-byte line, and just past one
-    (9, 512), (9, 513),                  # one wave per row, then two (backward)
-    (6, 2048), (6, 2049), (5, 5121),     # then four, with whole and ragged batches
+    (9, 512), (9, 513),                  # one wave per row, then four
+    (6, 2048), (6, 2049), (5, 5121),     # with whole and ragged batches
+    (2049, 513), (2049, 1537), (2049, 2047),  # many rows: one wave (forward), two (backward), one and four
     (3, 50257),
 ])
 @pytest.mark.parametrize("shift", [0, 1])
