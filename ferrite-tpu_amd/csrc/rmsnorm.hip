@@ -346,26 +346,11 @@ int group_of(int64_t dim, int unit) {
   const int64_t per = unit == 1 ? 16 : 32;
   return dim <= 64 * per ? 64 : dim <= 256 * per ? 256 : dim <= 512 * per ? 1024 : 0;
 }
-// Where all of a pass's streams fit the Infinity Cache (256 MB), the two-sweep kernels read their second
-// sweep from there, and with enough rows, a wave each, they are the better ones again for some pairs;
-// so they are for the shortest rows, which leave most of a group's lanes idle. us, two sweeps / groups:
-//   add+norm bf16 8192 x 1110 20 / 27, 32768 x 1110 76 / 78, 2048 x 4098 38 / 31
-//   f32 65536 x 130 27 / 37, 131072 x 150 84 / 75, 65536 x 34 14 / 18; norm bf16 8192 x 4098 43 / 59
-//   backward f32 32768 x 420 73 / 86, 8192 x 1026 52 / 47; bf16 32768 x 700 68 / 78
-bool cached(int streams, int64_t rows, int64_t dim, int esize) { return streams * rows * dim * esize <= (int64_t)272 << 20; }
-bool group_wins(int esize, int unit, int64_t rows, int64_t dim, bool residual) {
-  if (dim <= 64) return false;
-  if (unit == 2 && rows >= 4096 && cached(residual ? 4 : 2, rows, dim, esize)) {
-    if (residual && (esize == 4 ? dim <= 400 || (dim > 1024 && dim <= 2048) : dim > 1024 && rows * dim >= 1 << 23)) return false;
-    if (!residual && esize == 2 && dim > 4096 && rows >= 8192) return false;
-  }
+bool group_wins(int esize, int unit, int64_t dim, bool residual) {
   if (esize == 4 || unit == 8 || dim <= 256) return true;
   return unit == 2 ? residual || dim <= 1024 || dim > 2048 : dim > 4096;
 }
 bool group_wins_bwd(int esize, int unit, int64_t rows, int64_t dim) {
-  if (unit == 2 && rows >= 8192 && rows * dim >= 1 << 23 && cached(4, rows, dim, esize) &&
-      (esize == 4 ? dim > 128 && dim <= 1024 : dim > 400))
-    return false;
   if (esize == 4 || unit == 8 || dim <= 256) return true;
   return unit == 2 ? dim <= 2048 : rows * dim <= (int64_t)1 << 22;
 }
@@ -479,7 +464,7 @@ int launch(const void* x, const void* r, const void* w, void* h, void* y, int64_
     return aligned_to(x, bytes) && aligned_to(y, bytes) && (!RES || (aligned_to(r, bytes) && aligned_to(h, bytes)));
   };
   const int unit = unit_of(dim, all(16) && aligned_to(w, 16), all(2 * (int)sizeof(TX)));
-  const int group = group_wins((int)sizeof(TX), unit, rows, dim, RES) ? group_of(dim, unit) : 0;
+  const int group = group_wins((int)sizeof(TX), unit, dim, RES) ? group_of(dim, unit) : 0;
   if (group) {
     const int64_t per_block = group < 256 ? 256 / group : 1;
     // Persistent from eight workgroups of four waves per CU on.

@@ -274,7 +274,6 @@ def test_stream_read_and_fill_are_exact(dev, nbytes, blocks):
     (4, 4098, "f32"), (3, 4097, "bf16"), (700, 3001, "f32"),
     (3, 8200, "bf16"), (2, 16384, "f32"), (3, 8191, "f32"),  # 16 waves per row
     (3, 16392, "bf16"), (2, 8193, "f32"),                 # wider than any group: the two-sweep kernels
-    (70, 33, "bf16"), (4097, 130, "f32"), (8192, 1026, "bf16"),  # theirs too: short rows, and pairs that stay cached
     (5, 1000, "f32"),                                     # shifted: units of 8 become pairs or single elements
 ])
 @pytest.mark.parametrize("shift", [0, 1, 2])
