@@ -173,11 +173,19 @@ def _one_kernel_embedding(tok, pe, token, pos, dtype) -> bool:
 
 def _few_rows_head(y, emb) -> bool:
     """Whether the tied head's bf16 rows run on the few-rows kernel, which reads the embedding as it is. us
-    on one MI355X, that kernel / a bf16 copy of a float embedding and the library's product, V x d weights:
-    float   8 rows, 1000 x 512 5.7 / 8.4   32, 8192 x 2048 19.4 / 25.5   64, 8192 x 1024 15.6 / 19.3
-            40, 8192 x 2048 27.2 / 26.4    64, 32768 x 512 28.2 / 26.3
-    bf16    8, 8192 x 512 5.1 / 5.4        32, 1000 x 512 5.6 / 6.2      64, 256 x 512 7.3 / 10.0
-            64, 8192 x 512 8.0 / 7.2       8, 1000 x 1024 6.2 / 5.6      32, 300 x 129 6.5 / 5.7"""
+    on one MI355X, that kernel / a bf16 copy of a float embedding and the library's product, with the inputs
+    in the Infinity Cache, then from memory (rows, V x d weights); taken where neither is the slower:
+    float   8, 1000 x 512      5.7 / 8.4, 8.8 / 11.6
+            32, 8192 x 2048    19.4 / 25.5, 33.9 / 49.1
+            64, 8192 x 1024    15.6 / 19.3, 27.2 / 33.0
+            40, 8192 x 2048    27.2 / 26.4, 40.5 / 49.3
+            64, 32768 x 512    28.2 / 26.3, 44.4 / 47.5
+    bf16    8, 8192 x 512      5.1 / 5.4, 8.3 / 9.6
+            32, 1000 x 512     5.6 / 6.2, 7.9 / 12.4
+            64, 256 x 512      7.3 / 10.0, 10.1 / 17.0
+            64, 8192 x 512     8.0 / 7.2, 12.0 / 13.2
+            8, 1000 x 1024     6.2 / 5.6, 8.7 / 10.3
+            32, 300 x 129      6.5 / 5.7 cached"""
     rows, weights = y.shape[0], emb.numel()
     if y.dtype != torch.bfloat16 or rows > 64:
         return False
