@@ -180,19 +180,34 @@ def _few_rows_head(y, emb) -> bool:
             64, 8192 x 1024    15.6 / 19.3, 27.2 / 33.0
             40, 8192 x 2048    27.2 / 26.4, 40.5 / 49.3
             64, 32768 x 512    28.2 / 26.3, 44.4 / 47.5
-    bf16    8, 8192 x 512      5.1 / 5.4, 8.3 / 9.6
-            32, 1000 x 512     5.6 / 6.2, 7.9 / 12.4
+    bf16    8, 8192 x 512      3.5 / 3.9, 8.5 / 9.4
+            8, 256 x 960       4.4 / 8.3, 8.0 / 16.3
+            4, 1000 x 704      3.8 / 4.8, 7.4 / 10.2
+            16, 16384 x 904    6.9 / 7.7, 18.8 / 19.5
+            32, 2048 x 520     3.3 / 5.0, 8.0 / 11.2
             64, 256 x 512      7.3 / 10.0, 10.1 / 17.0
+    left    8, 1000 x 1024     4.7 / 4.1, 8.7 / 10.2
+            16, 8192 x 896     5.1 / 4.4, 11.4 / 11.9
+            32, 1000 x 704     4.9 / 4.4, 8.9 / 11.5
             64, 8192 x 512     8.0 / 7.2, 12.0 / 13.2
-            8, 1000 x 1024     6.2 / 5.6, 8.7 / 10.3
-            32, 300 x 129      6.5 / 5.7 cached"""
-    rows, weights = y.shape[0], emb.numel()
+            8, 4096 x 4096     11.2 / 9.8, 20.0 / 19.5
+            32, 300 x 129      6.5 / 5.7 cached
+    The library's few-row products of bf16 past 512 columns are fast where d is a multiple of 128 (up to 16
+    rows) or of 64 (beyond) and V more than 512."""
+    rows, (v, d), weights = y.shape[0], emb.shape, emb.numel()
     if y.dtype != torch.bfloat16 or rows > 64:
         return False
     if emb.dtype == torch.float32:
         return weights <= 1 << (24 if rows <= 32 else 23)
-    d = emb.shape[1]
-    return emb.dtype == torch.bfloat16 and d <= 512 and d % 8 == 0 and weights <= 1 << (22 if rows <= 32 else 17)
+    if emb.dtype != torch.bfloat16 or d % 8:
+        return False
+    if d <= 512:
+        return weights <= 1 << (22 if rows <= 32 else 17) or rows <= 16 and v <= 1 << 14
+    if v <= 512 and d < 1024:
+        return rows <= 32
+    if rows <= 16:
+        return v <= 1 << 14 and d <= 1216 and d % 128 != 0 and weights <= 1 << 24
+    return rows <= 32 and v <= 1 << 13 and d < 1024 and d % 64 != 0
 
 
 # The serving engine: captured prefill per bucket, one captured decode step.

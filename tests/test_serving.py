@@ -123,7 +123,10 @@ def test_few_rows_head_keeps_to_where_it_is_faster():
     cases = [(8, 1000, 512, f32, True), (32, 8192, 2048, f32, True), (33, 8192, 2048, f32, False),
              (64, 8192, 1024, f32, True), (65, 256, 256, f32, False), (1, 8193, 2048, f32, False),
              (32, 8192, 512, bf16, True), (33, 8192, 512, bf16, False), (8, 1000, 1024, bf16, False),
-             (64, 256, 512, bf16, True), (32, 300, 129, bf16, False), (8, 32768, 512, bf16, False), (8, 256, 256, torch.float16, False)]
+             (64, 256, 512, bf16, True), (32, 300, 129, bf16, False), (8, 32768, 512, bf16, False), (8, 256, 256, torch.float16, False),
+             (8, 256, 960, bf16, True), (4, 1000, 704, bf16, True), (16, 1000, 768, bf16, False), (16, 16384, 904, bf16, True),
+             (17, 16384, 904, bf16, False), (32, 2048, 520, bf16, True), (32, 1000, 704, bf16, False), (33, 256, 960, bf16, False),
+             (8, 8192, 1224, bf16, False), (8, 256, 1024, bf16, False)]
     for rows, v, d, dtype, takes in cases:
         emb = torch.empty(v, d, dtype=dtype, device="meta")
         assert _few_rows_head(torch.empty(rows, d, dtype=bf16, device="meta"), emb) == takes, (rows, v, d, dtype)
