@@ -127,12 +127,13 @@ __global__ __launch_bounds__(256) void embed_kernel(const int64_t* __restrict__ 
 // The token table's gradient of a small vocabulary: rows of dh summed by token. A tensor library
 // sorts the tokens and adds the many rows of each token one after another. Here a wave owns C
 // columns (a lane each) of a slice of the rows and adds every row into its own [vocab, C] table
-// in LDS, so nothing is sorted and each dh element is read once; a lane adds to its own column
-// in row order and the slices' tables are summed in slice order (deterministic). C is what a
-// 64 KB table leaves (two workgroups per CU): 64 up to 256 tokens, 16 up to 1024. Bound by the
-// chain of table updates in a wave: LDS atomics took 59 us for 16384 x 512 bf16 over 256 tokens,
-// reads and writes of two rows at a time 34. Training step of that size, tables' indexing in
-// torch / these kernels: 2894 / 2841 us.
+// in LDS, so nothing is sorted; a lane adds to its own column in row order and the slices' tables
+// are summed in slice order (deterministic). C is what a 64 KB table leaves (two workgroups per
+// CU): 64 up to 256 tokens, 32 up to 512 and 16 up to 1024, where the wave's 64 lanes load each dh
+// element two and four times. Bound by the chain of table updates in a wave: LDS atomics took 59 us
+// for 16384 x 512 bf16 over 256 tokens, reads and writes of two rows at a time 34; the sum of the
+// 64 slices' tables takes 17.7 more and the position table 4.8. Training step of that size, tables'
+// indexing in torch / these kernels: 2894 / 2841 us.
 constexpr int64_t kMostBlocks = 0xffffffff / 256;  // blocks of 256 threads: a launch has under 2^32 threads along x
 constexpr int kEmbedLds = 64 << 10;
 constexpr int64_t kEmbedVocab = 1024;

@@ -313,6 +313,7 @@ def _trunk(params, tokens, cfg: GPTConfig):
     if s > cfg.seq_len:
         raise ValueError(f"sequence {s} longer than cfg.seq_len={cfg.seq_len}")
     tok, pe = params["tok_emb"], params["pos_emb"]
+    # The residual stream's glue: on kernels where its other part, the add and norm, is.
     if cfg.norm == "pallas" and _one_kernel_embedding(tok, pe, tokens, cfg.dtype):
         h = _hip.autograd().embed_tokens(tokens, tok, pe, cfg.dtype)  # residual stream
     else:

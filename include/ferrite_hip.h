@@ -202,8 +202,9 @@ int ferrite_hip_matmul_ex(const void* x, const void* y, void* out, int64_t m, in
  *                           out <- bf16(bf16(op(x) @ op(y)) * gelu'(u))
  * gelu and gelu' are taken in f32 from the bf16-rounded values, as an elementwise
  * pass after the product computes them. Shapes the DMA-fed kernel takes apply
- * them in its store (or in the K split's reduction); others run the product and
- * then an elementwise pass.
+ * them in its store (or in the K split's reduction), products of up to 64 rows
+ * on the few-rows kernels in theirs; others run the product and then an
+ * elementwise pass.
  */
 int ferrite_hip_matmul_gelu(const void* x, const void* y, void* out, void* aux, int64_t m, int64_t n, int64_t k,
                             int x_t, int y_t, int mode, void* workspace, int64_t workspace_bytes, void* stream);
